@@ -1,8 +1,7 @@
-// gemm2.hip -- block-scaled MXFP4 x MXFP4 GEMM for large prefill shapes.
+// gemm2.hip -- block-scaled MXFP4 x MXFP4 GEMM for M > 16.
 //
 // y (M, N) fp32 = A (M, Kp) * W (N, Kp)^T, both operands packed E2M1 rows with
 // E8M0 32-block scales (the lin_pq contract, src/ext/mxfp4_decode.cu:135-170).
-// Used when Kp is a multiple of 256 and M > 16.
 //
 // * Workgroup tile BM x BN with NW waves in 2 (M) x NW/2 (N).  For large
 //   grids 256 x 256 with 8 waves: a wave owns 128 x 64 as 4 x 2
@@ -33,6 +32,15 @@
 // * Scales: BK/32 bytes per row per step, loaded the same way (4 bytes per
 //   lane) and permuted once per step (v_perm_b32) so that op_sel = ks selects
 //   the byte of K-substep ks.
+// * Kp not a multiple of 256 (RG): the lanes whose chunk lies past the row's
+//   end in the last step copy from an out-of-range offset, i.e. zeros, and
+//   those blocks' scale bytes are set to 127.  A row's scale bytes then start
+//   at any byte, so a step's copies take the four aligned dwords that hold its
+//   eight, and the operand reads shift them into place (two v_alignbyte): no
+//   unaligned copies, at twice the scale bytes (6 % of a step's copies).
+//   Measured on MI355X, 333 x 1000 x 2080: 20.9 us for the register-staged
+//   128 x 128 kernel that served these sizes before (24 workgroups, one
+//   memory round trip per K step), 9.2 us here.
 // * XCD-aware order: workgroup b runs on XCD b % 8; each XCD gets a compact
 //   block of tiles (a few tile rows by a few tile columns), so the A and W
 //   K-slabs of one step are fetched into that XCD's L2 once and shared.
@@ -42,14 +50,14 @@
 
 namespace {
 
-template <int BM, int BN, int BK, int NW>
+template <int BM, int BN, int BK, int NW, bool RG>
 struct Tile {
     static constexpr int WM = BM / 2;                     // rows per wave (2 waves along M)
     static constexpr int IM = WM / 32;                    // 32-row accumulator tiles per wave
     static constexpr int ROWB = BK / 2;                   // data bytes per row per step
     static constexpr int CPR = ROWB / 16;                 // 16-byte chunks per row
     static constexpr int RPB = 1024 / ROWB;               // rows per 1 KB copy block
-    static constexpr int SCB = BK / 32;                   // scale bytes per row per step
+    static constexpr int SCB = RG ? 16 : BK / 32;         // scale bytes copied per row per step
     static constexpr int KS = BK / 64;                    // MFMA K-substeps per step
     static constexpr int A_BYTES = BM * ROWB;
     static constexpr int W_BYTES = BN * ROWB;
@@ -67,6 +75,7 @@ struct Tile {
     static_assert(CPR == 4 || CPR == 8, "BK 128 or 256");
     static_assert(A_BYTES % (1024 * NW) == 0 && W_BYTES % (1024 * NW) == 0 && S_BYTES % 256 == 0, "copy split");
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
+    static_assert(!RG || BK == 256, "ragged K: 8 blocks per step");
 };
 
 struct G2Args {
@@ -105,20 +114,33 @@ __device__ __forceinline__ int swz_key(int r) {
 struct CopyState {
     v4u ra, rw, rsa, rsw;
     uint32_t va[2], vw[2];   // lane offset of A / W copies with an even / odd index
-    uint32_t vs;             // lane offset of scale copies
+    uint32_t vs;             // lane offset of scale copies (RG: of A's)
+    uint32_t vsw;            // RG: of W's
+    int ca[2], cw[2];        // RG: the lane's 32-block within the step, per copy parity
 };
 
-template <int BM, int BN, int BK, int NW>
+// RG: the byte at which the scale tensor starts within its first aligned dword.
+__device__ __forceinline__ uint32_t scale_delta(const uint8_t* p) { return (uint32_t)(uintptr_t)p & 3u; }
+
+template <int BM, int BN, int BK, int NW, bool RG>
 __device__ __forceinline__ CopyState copy_state(const G2Args& g, int m0, int n0) {
-    using T = Tile<BM, BN, BK, NW>;
+    using T = Tile<BM, BN, BK, NW, RG>;
     const int w = threadIdx.x >> 6;
     const int l = threadIdx.x & 63;
     const int64_t cbytes = g.Kp >> 1, nch = g.Kp >> 5;
     CopyState c;
-    c.ra = buf_rsrc(g.aq + m0 * cbytes, (int64_t)(g.M - m0) * cbytes);
-    c.rw = buf_rsrc(g.wp + n0 * cbytes, (int64_t)(g.N - n0) * cbytes);
-    c.rsa = buf_rsrc(g.as + m0 * nch, (int64_t)(g.M - m0) * nch);
-    c.rsw = buf_rsrc(g.ws + n0 * nch, (int64_t)(g.N - n0) * nch);
+    // (RG: no more than the tile's rows, so that a lane offset of 2^31 is out of range)
+    c.ra = buf_rsrc(g.aq + m0 * cbytes, (int64_t)(RG ? min(g.M - m0, BM) : g.M - m0) * cbytes);
+    c.rw = buf_rsrc(g.wp + n0 * cbytes, (int64_t)(RG ? min(g.N - n0, BN) : g.N - n0) * cbytes);
+    if constexpr (RG) {
+        // whole dwords (m0 and n0 are multiples of 64, so every tile starts at the tensor's own byte of a dword)
+        const int64_t da = scale_delta(g.as), dw = scale_delta(g.ws);
+        c.rsa = buf_rsrc(g.as + m0 * nch - da, ((int64_t)(g.M - m0) * nch + da + 3) & ~3ll);
+        c.rsw = buf_rsrc(g.ws + n0 * nch - dw, ((int64_t)(g.N - n0) * nch + dw + 3) & ~3ll);
+    } else {
+        c.rsa = buf_rsrc(g.as + m0 * nch, (int64_t)(g.M - m0) * nch);
+        c.rsw = buf_rsrc(g.ws + n0 * nch, (int64_t)(g.N - n0) * nch);
+    }
     const int lrow = l / T::CPR, slot = l % T::CPR;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
@@ -128,9 +150,17 @@ __device__ __forceinline__ CopyState copy_state(const G2Args& g, int m0, int n0)
         const int rw = (w * T::W_CP + p) * T::RPB + lrow;
         c.va[p] = (uint32_t)(ra * cbytes + ((slot ^ swz_key<T::CPR>(ra)) << 4)) - (uint32_t)(p * T::RPB * cbytes);
         c.vw[p] = (uint32_t)(rw * cbytes + ((slot ^ swz_key<T::CPR>(rw)) << 4)) - (uint32_t)(p * T::RPB * cbytes);
+        c.ca[p] = slot ^ swz_key<T::CPR>(ra);
+        c.cw[p] = slot ^ swz_key<T::CPR>(rw);
     }
     constexpr int LPR = T::SCB / 4;   // lanes per scale row
-    c.vs = (uint32_t)((l / LPR) * nch + 4 * (l % LPR));
+    if constexpr (RG) {
+        // the aligned dwords from the row's first byte on (a copy's first row is a multiple of 16)
+        c.vs = (((uint32_t)((l / LPR) * nch) + scale_delta(g.as)) & ~3u) + 4 * (l % LPR);
+        c.vsw = (((uint32_t)((l / LPR) * nch) + scale_delta(g.ws)) & ~3u) + 4 * (l % LPR);
+    } else {
+        c.vs = (uint32_t)((l / LPR) * nch + 4 * (l % LPR));
+    }
     return c;
 }
 
@@ -140,23 +170,26 @@ __device__ __forceinline__ CopyState copy_state(const G2Args& g, int m0, int n0)
 // the next step are spread over the MFMA substeps of this one (a wave issues
 // in order, so copies issued in one burst hold back its MFMAs while the
 // memory pipeline accepts them).
-template <int BM, int BN, int BK, int NW>
+template <int BM, int BN, int BK, int NW, bool RG>
 __device__ __forceinline__ void issue_part(const G2Args& g, const CopyState& c, uint32_t buf, int k0, int part) {
-    using T = Tile<BM, BN, BK, NW>;
+    using T = Tile<BM, BN, BK, NW, RG>;
     static_assert(T::A_CP % 2 == 0 && T::W_CP % 2 == 0, "even copy counts (swizzle key parity)");
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: scalar selects below
     const uint32_t cbytes = g.Kp >> 1, nch = g.Kp >> 5;
+    // RG: past the row's last block, an offset out of every range (zeros)
+    const int left = (int)nch - (k0 >> 5);
+    auto lane_off = [&](uint32_t v, int blk) { return RG && blk >= left ? 0x80000000u : v; };
 #pragma unroll
     for (int j = 0; j < T::A_CP; ++j) {
         if (j % T::KS != part) continue;
         const int blk = w * T::A_CP + j;   // c.va holds the wave's first block; soffset adds block j
-        dma16(c.va[j & 1], c.ra, (uint32_t)(j * T::RPB) * cbytes + (k0 >> 1), buf + blk * 1024);
+        dma16(lane_off(c.va[j & 1], c.ca[j & 1]), c.ra, (uint32_t)(j * T::RPB) * cbytes + (k0 >> 1), buf + blk * 1024);
     }
 #pragma unroll
     for (int j = 0; j < T::W_CP; ++j) {
         if ((T::A_CP + j) % T::KS != part) continue;
         const int blk = w * T::W_CP + j;
-        dma16(c.vw[j & 1], c.rw, (uint32_t)(j * T::RPB) * cbytes + (k0 >> 1), buf + T::A_BYTES + blk * 1024);
+        dma16(lane_off(c.vw[j & 1], c.cw[j & 1]), c.rw, (uint32_t)(j * T::RPB) * cbytes + (k0 >> 1), buf + T::A_BYTES + blk * 1024);
     }
     // scales: rows 0..BM-1 of A then 0..BN-1 of W, SCB bytes each, 4 bytes a
     // lane; waves past the last copy rewrite an earlier one (same bytes)
@@ -172,15 +205,15 @@ __device__ __forceinline__ void issue_part(const G2Args& g, const CopyState& c, 
         rs.y = __builtin_amdgcn_readfirstlane(is_a ? c.rsa.y : c.rsw.y);
         rs.z = __builtin_amdgcn_readfirstlane(is_a ? c.rsa.z : c.rsw.z);
         rs.w = 0x00020000u;
-        dma4(c.vs, rs, (uint32_t)((is_a ? row0 : row0 - BM)) * nch + (k0 >> 5),
+        dma4(RG && !is_a ? c.vsw : c.vs, rs, (uint32_t)((is_a ? row0 : row0 - BM)) * nch + (k0 >> 5),
              buf + T::A_BYTES + T::W_BYTES + q * 256);
     }
 }
 
-template <int BM, int BN, int BK, int NW>
+template <int BM, int BN, int BK, int NW, bool RG>
 __device__ __forceinline__ void issue_stage(const G2Args& g, const CopyState& c, uint32_t buf, int k0) {
 #pragma unroll
-    for (int q = 0; q < Tile<BM, BN, BK, NW>::KS; ++q) issue_part<BM, BN, BK, NW>(g, c, buf, k0, q);
+    for (int q = 0; q < Tile<BM, BN, BK, NW, RG>::KS; ++q) issue_part<BM, BN, BK, NW, RG>(g, c, buf, k0, q);
 }
 
 template <int OP>
@@ -190,10 +223,18 @@ __device__ __forceinline__ mx::v16f mfma32(uint4 a, uint4 b, mx::v16f c, uint32_
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, c, 4, 4, OP, (int)sa, OP, (int)sb);
 }
 
-// Scale word of this lane: byte ks = block 2*ks + h of the step.
-template <int SCB>
-__device__ __forceinline__ uint32_t scale_word(const uint8_t* srow, int h) {
-    if constexpr (SCB == 8) {
+// Scale word of this lane: byte ks = block 2*ks + h of the step.  RG: the
+// step's eight bytes start `shift` bytes into the row's 16; `keep` has the
+// bytes of blocks inside the row set, the others become 127.
+template <int SCB, bool RG>
+__device__ __forceinline__ uint32_t scale_word(const uint8_t* srow, int h, uint32_t shift, uint32_t keep) {
+    if constexpr (RG) {
+        const uint2 v = *reinterpret_cast<const uint2*>(srow);
+        const uint32_t v2 = *reinterpret_cast<const uint32_t*>(srow + 8);
+        const uint32_t lo = __builtin_amdgcn_alignbyte(v.y, v.x, shift), hi = __builtin_amdgcn_alignbyte(v2, v.y, shift);
+        const uint32_t w = __builtin_amdgcn_perm(hi, lo, h ? 0x07050301u : 0x06040200u);
+        return (w & keep) | (0x7F7F7F7Fu & ~keep);
+    } else if constexpr (SCB == 8) {
         const uint2 v = *reinterpret_cast<const uint2*>(srow);
         return __builtin_amdgcn_perm(v.y, v.x, h ? 0x07050301u : 0x06040200u);
     } else {
@@ -206,10 +247,10 @@ __device__ __forceinline__ uint32_t scale_word(const uint8_t* srow, int h) {
 // wm*128 + i*32 + lr and wn*BN/4 + j*32 + lr, differ from lr by multiples of
 // 16, so their swizzle key is swz_key(lr): one LDS address per operand and
 // K-substep, the row offsets are immediates.
-template <int BM, int BN, int BK, int NW>
-__device__ __forceinline__ void mfma_step(const uint8_t* cur, mx::v16f (&acc)[Tile<BM, BN, BK, NW>::IM][Tile<BM, BN, BK, NW>::TN], const G2Args& g,
-                                          const CopyState& cs, uint32_t nxt, int k_next) {
-    using T = Tile<BM, BN, BK, NW>;
+template <int BM, int BN, int BK, int NW, bool RG>
+__device__ __forceinline__ void mfma_step(const uint8_t* cur, mx::v16f (&acc)[Tile<BM, BN, BK, NW, RG>::IM][Tile<BM, BN, BK, NW, RG>::TN], const G2Args& g,
+                                          const CopyState& cs, uint32_t nxt, int k_next, int k_cur) {
+    using T = Tile<BM, BN, BK, NW, RG>;
     constexpr int TN = T::TN;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -222,10 +263,20 @@ __device__ __forceinline__ void mfma_step(const uint8_t* cur, mx::v16f (&acc)[Ti
     const uint8_t* lsa = cur + T::A_BYTES + T::W_BYTES + (wm * T::WM + lr) * T::SCB;
     const uint8_t* lsw = cur + T::A_BYTES + T::W_BYTES + BM * T::SCB + (wn * T::WCOLS + lr) * T::SCB;
     uint32_t sa[T::IM], sb[TN];
+    uint32_t sha = 0, shw = 0, keep = 0xFFFFFFFFu;
+    if constexpr (RG) {
+        // rows a multiple of 32 apart share their shift
+        sha = (uint32_t)(lr * (g.Kp >> 5)) + scale_delta(g.as);
+        shw = (uint32_t)(lr * (g.Kp >> 5)) + scale_delta(g.ws);
+        sha &= 3u;
+        shw &= 3u;
+        const int in = ((g.Kp - k_cur) >> 5) + 1 - h;   // blocks 2 ks + h < left: ks < in / 2
+        keep = in >= 8 ? 0xFFFFFFFFu : (1u << (4 * (in & ~1))) - 1u;
+    }
 #pragma unroll
-    for (int i = 0; i < T::IM; ++i) sa[i] = scale_word<T::SCB>(lsa + i * 32 * T::SCB, h);
+    for (int i = 0; i < T::IM; ++i) sa[i] = scale_word<T::SCB, RG>(lsa + i * 32 * T::SCB, h, sha, keep);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) sb[j] = scale_word<T::SCB>(lsw + j * 32 * T::SCB, h);
+    for (int j = 0; j < TN; ++j) sb[j] = scale_word<T::SCB, RG>(lsw + j * 32 * T::SCB, h, shw, keep);
     // operand registers of two substeps: the reads of substep ks+1 are issued
     // before the MFMAs of substep ks, so their LDS latency hides under them
     uint4 af[2][T::IM], bf[2][TN];
@@ -242,7 +293,7 @@ __device__ __forceinline__ void mfma_step(const uint8_t* cur, mx::v16f (&acc)[Ti
         // keep each substep's copies, operand reads and MFMAs together (the
         // scheduler would otherwise hoist every copy ahead of the MFMAs)
         __builtin_amdgcn_sched_barrier(0);
-        issue_part<BM, BN, BK, NW>(g, cs, nxt, k_next, ks);
+        issue_part<BM, BN, BK, NW, RG>(g, cs, nxt, k_next, ks);
         if (ks + 1 < T::KS) load(ks + 1, (ks + 1) & 1);
         const int r = ks & 1;
 #pragma unroll
@@ -257,9 +308,9 @@ __device__ __forceinline__ void mfma_step(const uint8_t* cur, mx::v16f (&acc)[Ti
     }
 }
 
-template <int BM, int BN, int BK, int NSTAGE, int NW>
+template <int BM, int BN, int BK, int NSTAGE, int NW, bool RG>
 __global__ __launch_bounds__(64 * NW, 1) void gemm2_kernel(G2Args g) {
-    using T = Tile<BM, BN, BK, NW>;
+    using T = Tile<BM, BN, BK, NW, RG>;
     constexpr int TN = T::TN;
     static_assert(NSTAGE >= 2 && NSTAGE * T::STAGE <= 160 * 1024, "LDS ring");
     __shared__ __align__(16) uint8_t ring[NSTAGE * T::STAGE];
@@ -282,7 +333,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm2_kernel(G2Args g) {
     const int wm = wave / T::WN_W, wn = wave % T::WN_W;
     const int lr = lane & 31;
     const int h = lane >> 5;
-    const int nsteps = g.Kp / BK;
+    const int nsteps = RG ? (g.Kp + BK - 1) / BK : g.Kp / BK;
 
     mx::v16f acc[T::IM][TN];
 #pragma unroll
@@ -292,10 +343,10 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm2_kernel(G2Args g) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    const CopyState cs = copy_state<BM, BN, BK, NW>(g, m0, n0);
+    const CopyState cs = copy_state<BM, BN, BK, NW, RG>(g, m0, n0);
     const uint32_t ring_lds = __builtin_amdgcn_readfirstlane(lds_addr(ring));   // LDS byte address of the ring
 #pragma unroll
-    for (int s = 0; s < NSTAGE - 1; ++s) issue_stage<BM, BN, BK, NW>(g, cs, ring_lds + s * T::STAGE, min(s, nsteps - 1) * BK);
+    for (int s = 0; s < NSTAGE - 1; ++s) issue_stage<BM, BN, BK, NW, RG>(g, cs, ring_lds + s * T::STAGE, min(s, nsteps - 1) * BK);
 
     for (int it0 = 0; it0 < nsteps; it0 += NSTAGE) {
 #pragma unroll
@@ -313,8 +364,8 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm2_kernel(G2Args g) {
                 asm volatile("" ::: "memory");
                 // MFMAs on this step's stage; the stage step it-1 used is
                 // refilled with step it+NSTAGE-1, spread over the substeps
-                mfma_step<BM, BN, BK, NW>(ring + s * T::STAGE, acc, g, cs, ring_lds + ((s + NSTAGE - 1) % NSTAGE) * T::STAGE,
-                                  min(it + NSTAGE - 1, nsteps - 1) * BK);
+                mfma_step<BM, BN, BK, NW, RG>(ring + s * T::STAGE, acc, g, cs, ring_lds + ((s + NSTAGE - 1) % NSTAGE) * T::STAGE,
+                                  min(it + NSTAGE - 1, nsteps - 1) * BK, it * BK);
             }
         }
     }
@@ -366,45 +417,49 @@ void xcd_blocks(G2Args& g) {
 }  // namespace
 
 namespace mxh {
-// Any M > 16 with Kp a multiple of 256 (the buffer descriptors address each
-// operand with 32-bit byte offsets, hence the size bound).
-bool lin_pq_gemm2_supported(int M, int N, int Kp) {
-    const bool fits = (int64_t)M * (Kp / 2) < (1ll << 32) && (int64_t)N * (Kp / 2) < (1ll << 32);
-    return M > 16 && N > 0 && Kp >= 256 && (Kp % 256) == 0 && fits;
-}
+// Any M > 16 (a tile's rows are addressed with 32-bit byte offsets, hence the
+// bound on Kp; longer rows take the GEMV in chunks of 16 rows).
+bool lin_pq_gemm2_supported(int M, int N, int Kp) { return M > 16 && N > 0 && Kp > 0 && Kp <= (1 << 22); }
 
-template <int BM, int BN, int BK, int NSTAGE, int NW>
+template <int BM, int BN, int BK, int NSTAGE, int NW, bool RG>
 int launch_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y, int M, int N,
                  int Kp, hipStream_t st) {
-    MXH_REQUIRE(Kp % BK == 0, "lin_pq_gemm2: Kp=%d is not a multiple of %d", Kp, BK);
+    MXH_REQUIRE(RG || Kp % BK == 0, "lin_pq_gemm2: Kp=%d is not a multiple of %d", Kp, BK);
     G2Args g{xq, xsc, wp, wsc, y, M, N, Kp, 0, 0, 0, 0, 0, 0};
     g.tiles_m = (M + BM - 1) / BM;
     g.tiles_n = (N + BN - 1) / BN;
     xcd_blocks(g);
-    hipLaunchKernelGGL((gemm2_kernel<BM, BN, BK, NSTAGE, NW>), dim3(8 * g.per_xcd), dim3(64 * NW), 0, st, g);
+    hipLaunchKernelGGL((gemm2_kernel<BM, BN, BK, NSTAGE, NW, RG>), dim3(8 * g.per_xcd), dim3(64 * NW), 0, st, g);
     return launch_status("lin_pq_gemm2");
 }
 
-int lin_pq_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y,
-                 int M, int N, int Kp, hipStream_t st) {
-    MXH_REQUIRE(((uintptr_t)xq & 15) == 0 && ((uintptr_t)wp & 15) == 0,
-                "lin_pq: packed operands must be 16-byte aligned");
-    MXH_REQUIRE(((uintptr_t)xsc & 3) == 0 && ((uintptr_t)wsc & 3) == 0,
-                "lin_pq: scale rows must be 4-byte aligned");
+template <bool RG>
+int pick_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y, int M, int N,
+               int Kp, hipStream_t st) {
     // Tile by grid size: 256 x 256 (2 stages) when it gives at least 128
     // tiles; else 128 x 128 (4 stages) when that gives at least 192; else
     // 64 x 64 with 8 stages, i.e. up to 7 K-steps of copies in flight, so a
     // small grid pays about one memory latency instead of one per K-step --
     // or with 4 stages (two workgroups per CU) when one per CU would take
     // two rounds.  Measured on MI355X: 512 x 1536 x 2048 in 6.5 us against
-    // 11.1 us for the 128 x 128 register-staged GEMM; all tiles give the same
-    // bits (the same MFMA chain per output).
+    // 11.1 us for 128 x 128 tiles; all tiles give the same bits (the same
+    // MFMA chain per output).
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-    if (t256 >= 128) return launch_gemm2<256, 256, 256, 2, 8>(xq, xsc, wp, wsc, y, M, N, Kp, st);
-    if (t128 >= 192) return launch_gemm2<128, 128, 256, 4, 4>(xq, xsc, wp, wsc, y, M, N, Kp, st);
-    if (t64 > 256) return launch_gemm2<64, 64, 256, 4, 4>(xq, xsc, wp, wsc, y, M, N, Kp, st);
-    return launch_gemm2<64, 64, 256, 8, 4>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    if (t256 >= 128) return launch_gemm2<256, 256, 256, 2, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    if (t128 >= 192) return launch_gemm2<128, 128, 256, 4, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    if (t64 > 256) return launch_gemm2<64, 64, 256, 4, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    return launch_gemm2<64, 64, 256, 8, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+}
+
+int lin_pq_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y,
+                 int M, int N, int Kp, hipStream_t st) {
+    MXH_REQUIRE(((uintptr_t)xq & 15) == 0 && ((uintptr_t)wp & 15) == 0,
+                "lin_pq: packed operands must be 16-byte aligned");
+    if (Kp % 256 != 0) return pick_gemm2<true>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    MXH_REQUIRE(((uintptr_t)xsc & 3) == 0 && ((uintptr_t)wsc & 3) == 0,
+                "lin_pq: scale rows must be 4-byte aligned");
+    return pick_gemm2<false>(xq, xsc, wp, wsc, y, M, N, Kp, st);
 }
 }  // namespace mxh

@@ -15,9 +15,6 @@ int quantize_rows_impl(const void* x, int src_dtype, int round_to_f16, int64_t l
                        int Kp, uint8_t* q, uint8_t* s, hipStream_t st);
 int lin_pq_gemv(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc,
                 float* y, int M, int N, int K, int Kp, hipStream_t st);
-int lin_pq_gemm(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc,
-                float* y, int M, int N, int Kp, hipStream_t st);
-bool lin_pq_gemm_supported(int M, int N, int Kp);
 int lin_pq_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc,
                  float* y, int M, int N, int Kp, hipStream_t st);
 bool lin_pq_gemm2_supported(int M, int N, int Kp);
@@ -37,8 +34,6 @@ extern "C" int mxfp4_lin_pq(const uint8_t* xq, const uint8_t* xsc, const uint8_t
     hipStream_t st = mxh::as_stream(stream);
     if (M > kGemvMaxM && mxh::lin_pq_gemm2_supported(M, N, Kp))
         return mxh::lin_pq_gemm2(xq, xsc, wp, wsc, y, M, N, Kp, st);
-    if (M > kGemvMaxM && mxh::lin_pq_gemm_supported(M, N, Kp))
-        return mxh::lin_pq_gemm(xq, xsc, wp, wsc, y, M, N, Kp, st);
     return mxh::lin_pq_gemv(xq, xsc, wp, wsc, y, M, N, K, Kp, st);
 }
 

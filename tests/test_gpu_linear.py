@@ -57,6 +57,36 @@ FWD_SHAPES = [(16, 8, 64), (16, 8, 100), (16, 8, 40), (1, 8, 64), (1, 32, 64), (
               (32, 32, 64), (8, 64, 2048), (1, 768, 2048), (8, 2048, 768), (2048, 2048, 768)]
 
 
+# M > 16 with Kp % 256 != 0: one block and one short of a step, scale rows that start at any byte of a dword,
+# a tail after full steps on each tile size (64 x 64 in eight and four stages, 128 x 128, 256 x 256)
+RAGGED_SHAPES = [(17, 33, 32), (65, 127, 224), (333, 1000, 2080), (100, 129, 1312 + 256), (200, 64, 2048 + 96),
+                 (1100, 900, 544), (1500, 2100, 800), (3000, 3100, 288)]
+
+
+@pytest.mark.parametrize("M,N,K", RAGGED_SHAPES)
+def test_lin_pq_ragged_k_vs_oracle(dext, M, N, K):
+    test_lin_pq_vs_oracle(dext, M, N, K)
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_lin_pq_ragged_scales_at_any_byte(dext, shift):
+    """Scale tensors that start inside a dword give the bits of aligned ones."""
+    M, N, K = 70, 150, 1120
+    wp, wsc, _, _ = _w(dext, N, K, seed=71)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(72)
+    xq, xs = dext.prequant(torch.randn((M, K), generator=g, device=DEV).bfloat16())
+
+    def moved(t, by):
+        buf = torch.zeros(t.numel() + 8, dtype=torch.uint8, device=DEV)
+        v = buf[by:by + t.numel()].view(t.shape)
+        v.copy_(t)
+        return v
+
+    want = dext.lin_pq(xq, xs, wp, wsc, M, N, K)
+    assert torch.equal(dext.lin_pq(xq, moved(xs, shift), wp, moved(wsc, 4 - shift), M, N, K), want)
+
+
 @pytest.mark.parametrize("M,N,K", FWD_SHAPES)
 @pytest.mark.parametrize("xdt", [torch.float16, torch.bfloat16])
 def test_forward_vs_oracle(lext, M, N, K, xdt):
