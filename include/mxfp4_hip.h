@@ -151,7 +151,7 @@ int mxfp4_moe_combine(const float* yd, int ystride, const float* w, int E,
  *   o          f32 (M, Hq, D): softmax(q.k / sqrt(D)) . v
  *   workspace  16-byte aligned device memory of
  *              mxfp4_attn_decode_workspace_size(M, Hq, max_pos) bytes (the
- *              per-64-position softmax partials; nothing persists)
+ *              softmax partials; nothing persists)
  */
 size_t mxfp4_attn_decode_workspace_size(int M, int Hq, int max_pos);
 int mxfp4_attn_decode(const void* q, const uint8_t* kvk, const uint8_t* kvv, const int32_t* dpos,

@@ -16,6 +16,7 @@
 //                        chunk's softmax statistics and its partial weighted
 //                        sum of V (V rows read once for the group) -> one
 //                        record per (token, head, chunk) in the workspace.
+//   attn_split.hip       the same for several tokens over a long cache.
 //   attn_final_kernel    workgroup (query head, token): merges the records
 //                        (split softmax: rescale by exp(m_c - max)); fp32
 //                        output and/or its bf16 -> MXFP4 rows.
@@ -28,6 +29,7 @@
 // exponent-15 codes read as 56 * (8 + m).
 #include "attn_merge.h"
 #include "attn_partial.h"
+#include "attn_split.h"
 #include "head_rope.h"
 #include "mx_device.h"
 #include "mx_host.h"
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(256) void attn_final_kernel(const float* __restrict
                                                          uint8_t* __restrict__ oq, uint8_t* __restrict__ os,
                                                          const int32_t* __restrict__ dpos, int Hq, int max_pos,
                                                          int nchunk) {
-    const int h = blockIdx.x, m = blockIdx.y, lane = threadIdx.x & 63;
+    const int h = blockIdx.x, m = blockIdx.y;
     const int pos = *dpos + m;
     if (pos < 0 || pos >= max_pos) return;
     const int n = pos / kChunk + 1;            // chunks holding positions 0..pos
@@ -74,14 +76,7 @@ __global__ __launch_bounds__(256) void attn_final_kernel(const float* __restrict
     __shared__ am::MergeLds lds;
     float r0, r1;
     if (!am::merge_head(rec, n, lds, r0, r1)) return;
-    if (o) *reinterpret_cast<float2*>(o + ((int64_t)m * Hq + h) * kD + 2 * lane) = make_float2(r0, r1);
-    if (oq) {
-        uint32_t byte, code;
-        am::quant_head_row(r0, r1, byte, code);
-        const int64_t rowq = (int64_t)m * (Hq * kD / 2) + h * (kD / 2);
-        if ((lane & 3) == 0) *reinterpret_cast<uint32_t*>(oq + rowq + lane) = byte;
-        if ((lane & 15) == 0) os[(int64_t)m * (Hq * kD / 32) + h * (kD / 32) + lane / 16] = (uint8_t)code;
-    }
+    am::write_head(o, oq, os, m, h, Hq, r0, r1);
 }
 
 __global__ __launch_bounds__(256) void kv_write_kernel(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
@@ -127,6 +122,26 @@ int launch_attn(const void* q, const uint8_t* kvk, const uint8_t* kvv, const int
     MXH_REQUIRE(workspace_bytes >= mxfp4_attn_decode_workspace_size(M, Hq, max_pos) && ((uintptr_t)workspace & 15) == 0,
                 "attn_decode: workspace must be 16-byte aligned and hold mxfp4_attn_decode_workspace_size bytes");
     const int G = Hq / Hkv;
+    // Several tokens over a cache of more than 64 chunks: the context-split
+    // kernel (attn_split.hip) for every entry, so that they go on agreeing bit
+    // for bit.  The chunk pass writes a record per token, head and 64 positions
+    // there (55 MB at 9 tokens and 23001 positions, more than the cache's 24)
+    // and decodes each byte for 4 tokens at a time.  One token stays on chunks,
+    // whose records the layer launch merges, and so does a short cache, where
+    // both wait on latency: 4096 positions, 1 token 9.8 against 8.4 us, 9 tokens
+    // 19.6 against 15.4; 23001 positions, 4 tokens 29.5 against 19.2, 9 tokens
+    // 54.4 against 25.2, 16 tokens 73.6 against 34.0.
+    if (M > 1 && max_pos > 64 * kChunk && merge && G <= 16 && (G & (G - 1)) == 0) {
+        if constexpr (FUSED) {
+            // the head norm, RoPE and KV write as their own launch, q past the records
+            void* qb = static_cast<uint8_t*>(workspace) + mxh::attn_split_record_bytes(M, Hq, Hkv, max_pos);
+            const int rc = mxfp4_qk_norm_rope_kv(fz.qkv, fz.qw, fz.kw, fz.eps, fz.theta, dpos, M, Hq, Hkv, D, qb,
+                                                 fz.kvk_w, fz.kvv_w, max_pos, fz.codec, st);
+            if (rc != MXFP4_OK) return rc;
+            q = qb;
+        }
+        return mxh::attn_split(q, kvk, kvv, dpos, sc, o, oq, os, M, Hq, Hkv, max_pos, workspace, st);
+    }
     const int nchunk = (max_pos + kChunk - 1) / kChunk;
     const float invsqrt = 1.0f / sqrtf((float)D);
     // row tiles of 16 query rows per workgroup, at most 2: more token groups

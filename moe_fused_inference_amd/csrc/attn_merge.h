@@ -33,9 +33,12 @@ struct MergeLds {
 // (m_c, l_c) (a thread per chunk), pass 2 sums the column records with all
 // loads in flight.  The four phases meet in LDS.  Returns true in wave 0,
 // whose lane l then holds o[2l], o[2l+1] in r0, r1; the other waves return
-// false and must not wait at a barrier afterwards.
+// false and must not wait at a barrier afterwards.  LOG2: the records'
+// maxima are in base 2 (the sums of exp2(s - m_c)).
+template <bool LOG2 = false>
 __device__ __forceinline__ bool merge_head(const float* rec, int n, MergeLds& s, float& r0, float& r1) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    auto weight = [](float d) { return LOG2 ? __builtin_amdgcn_exp2f(d) : expf(d); };
     if (n <= 64) {
         constexpr int kF = 16;
         float2 st[kF], cs[kF];
@@ -60,7 +63,7 @@ __device__ __forceinline__ bool merge_head(const float* rec, int n, MergeLds& s,
 #pragma unroll
         for (int i = 0; i < kF; ++i) {
             if (wave + 4 * i < n) {
-                const float w = expf(st[i].x - gm);
+                const float w = weight(st[i].x - gm);
                 den = fmaf(w, st[i].y, den);
                 num.x = fmaf(w, cs[i].x, num.x);
                 num.y = fmaf(w, cs[i].y, num.y);
@@ -101,7 +104,7 @@ __device__ __forceinline__ bool merge_head(const float* rec, int n, MergeLds& s,
     for (int i = 0; i < kPer; ++i) {
         const int c = i * 256 + tid;
         if (c < n) {
-            const float w = expf(mc[i] - gm);
+            const float w = weight(mc[i] - gm);
             s.cw[c] = w;
             den = fmaf(w, lc[i], den);
         }
@@ -145,6 +148,20 @@ __device__ __forceinline__ void quant_head_row(float r0, float r1, uint32_t& byt
     byte |= (uint32_t)mx::dpp<mx::kDppQuadNext1>((int)byte) << 8;    // lane 4j: bytes of 4j..4j+3
     byte |= (uint32_t)mx::dpp<mx::kDppQuadNext2>((int)byte) << 16;
     bytes4 = byte;
+}
+
+// Wave 0's head row (r0, r1 as merge_head leaves them) of token m to o (M, Hq,
+// D) fp32 and / or the MXFP4 rows oq / os of bf16(o); either may be null.
+__device__ __forceinline__ void write_head(float* o, uint8_t* oq, uint8_t* os, int m, int h, int Hq, float r0, float r1) {
+    const int lane = threadIdx.x & 63;
+    if (o) *reinterpret_cast<float2*>(o + ((int64_t)m * Hq + h) * kD + 2 * lane) = make_float2(r0, r1);
+    if (oq) {
+        uint32_t byte, code;
+        quant_head_row(r0, r1, byte, code);
+        const int64_t rowq = (int64_t)m * (Hq * kD / 2) + h * (kD / 2);
+        if ((lane & 3) == 0) *reinterpret_cast<uint32_t*>(oq + rowq + lane) = byte;
+        if ((lane & 15) == 0) os[(int64_t)m * (Hq * kD / 32) + h * (kD / 32) + lane / 16] = (uint8_t)code;
+    }
 }
 
 }  // namespace am

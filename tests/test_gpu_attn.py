@@ -181,3 +181,47 @@ def test_attn_decode_mx_quantized_output(M, Hq, Hkv, max_pos, base):
         assert np.array_equal(np_(oq)[live], rq[live]) and np.array_equal(np_(os_)[live], rs[live]), f"call {call}"
         ref, _ = attn.attn_decode_ref(q.float().cpu().numpy(), np_(kvk), np_(kvv), base)
         assert_close(np_(o2)[live], ref[live], what=f"attn_decode_mx call {call}")
+
+
+# several tokens over a cache of more than 4096 positions: one, two and three row tiles and more than one row group,
+# a split's edges (32- and 128-position multiples and their neighbours), a context far shorter than the cache, score rows
+# that are not 16-byte aligned (max_pos % 4 != 0), positions outside the cache
+@pytest.mark.parametrize("M,Hq,Hkv,max_pos,base", [(2, 4, 4, 4100, 4098), (2, 32, 4, 4097, 31), (3, 32, 4, 8192, 127),
+                                                   (5, 32, 4, 5001, 4996), (6, 8, 8, 4224, 4223), (9, 32, 4, 6000, 5000),
+                                                   (13, 16, 1, 4160, 1000), (16, 32, 2, 4352, 32), (2, 16, 16, 4104, -1),
+                                                   (300, 2, 2, 4500, 4300)])
+def test_attn_decode_split_vs_oracle(dext, M, Hq, Hkv, max_pos, base):
+    """The context-split path: output and raw scores against the oracle; sc
+    untouched past a token's position; a V cache that starts at any dword
+    gives the same bits."""
+    rng = np.random.default_rng(M * 11 + max_pos + base)
+    kvk_np, kvv_np = _cache(rng, max_pos, Hkv, 128), _cache(rng, max_pos, Hkv, 128)
+    kvk_np[5::701] = _cache(rng, max_pos, Hkv, 128, 150.0)[5::701]      # exponent field 15 among them
+    kvv_np[3::97] = _cache(rng, max_pos, Hkv, 128, 300.0)[3::97]
+    q = _bf16(rng.standard_normal((M, Hq, 128)))
+    sc = torch.full((M, Hq, max_pos), float("nan"), dtype=torch.float32, device=DEV)
+    kvk, kvv = torch.from_numpy(kvk_np).to(DEV), torch.from_numpy(kvv_np).to(DEV)
+    dpos = torch.tensor([base], dtype=torch.int32, device=DEV)
+    o = dext.attn_decode(q.to(DEV), kvk, kvv, dpos, sc, M)
+    moved = torch.empty(kvv.numel() + 16, dtype=torch.uint8, device=DEV)[4:4 + kvv.numel()].view(kvv.shape)
+    moved.copy_(kvv)
+    o4 = dext.attn_decode(q.to(DEV), kvk, moved, dpos, torch.empty_like(sc), M)
+    torch.cuda.synchronize()
+    ref, scores = attn.attn_decode_ref(q.float().numpy(), kvk_np, kvv_np, base)
+    live = [m for m in range(M) if 0 <= base + m < max_pos]
+    # 21 bits of each probability, fp32 sums: ten times what 32 bits leave
+    assert_close(np_(o)[live], ref[live], what=f"attn split M={M} Hq={Hq} Hkv={Hkv} base={base}", rel_max=1e-5)
+    assert torch.equal(o[live], o4[live])
+    for m in live[:20]:
+        S = base + m + 1
+        err = np.abs(np_(sc[m, :, :S]).astype(np.float64) - scores[m]).max() / np.abs(scores[m]).max()
+        assert err <= 1e-5, (m, err)
+    assert torch.isnan(sc[live[0], :, base + live[0] + 1:]).all()
+
+
+@pytest.mark.parametrize("codec", [0, 1])
+def test_attn_decode_fused_split_matches_two_ops(codec):
+    """Past 4096 positions mxfp4_attn_decode_fused with several tokens still
+    equals qk_norm_rope_kv followed by attn_decode_mx bit for bit."""
+    from tests.test_gpu_decode_step import test_attn_decode_fused_matches_two_ops as check
+    check(5, 32, 4, 6001, 5998, codec)
