@@ -23,6 +23,7 @@
 //   prefetch).
 // * The pointer tables travel by value in the kernel arguments, replacing the
 //   reference's host-blocking H2D table copy (src/ext/mxfp4_decode_binding.cpp:58).
+#include "lds_dma.h"
 #include "mx_device.h"
 #include "mx_host.h"
 
@@ -438,6 +439,135 @@ __global__ __launch_bounds__(64 * R * S) void lin_small_kernel(const uint8_t* __
     }
 }
 
+// The same for a weight of many rows (the vocabulary head): one workgroup per
+// CU, whose four waves each walk row tiles t, t + waves, ... with the weight
+// streaming through a ring of their own in LDS.
+//  * What bounds it is the weight stream.  With a tile per wave (the kernel
+//    above) a wave has two 4 KB segments in flight, in 64-byte pieces of 16
+//    rows, starts with a latency and ends with one; here the copies (global ->
+//    LDS, no registers) run three stages of 16 rows x 512 bytes ahead without a
+//    break, in pieces of 512 contiguous bytes, ~100 KB per CU.
+//  * The activation rows sit in LDS (rows past M are zeros), the ring's
+//    16-byte chunks under an XOR with the row, so that the 16 rows of an
+//    operand read hit 16 bank groups.  No barrier in the loop: a wave waits
+//    for its own copies only.  The output's stores count in the same counter,
+//    so the wait behind them asks for a little more than the stage.
+//  * The MFMA chain of an output is lin_small_kernel<4, 1>'s: the same bits.
+// Measured on MI355X, 151936 x 2048 from HBM, M = 8: 42.5 us for the tile per
+// wave, 34.5 us (4.8 TB/s) here.
+constexpr int kStRows = 16, kStK = 1024;                    // a stage: weight rows, K
+constexpr int kStRowB = kStK / 2, kStNch = kStK / 32;       // bytes, 32-blocks per row
+constexpr int kStData = kStRows * kStRowB;                  // 8 KB
+constexpr int kStBytes = kStData + kStRows * kStNch;
+constexpr int kStCopies = kStData / 1024 + 1;               // copies per stage
+
+__host__ __device__ constexpr int st_arow(int Kp) { return Kp / 2 + 16; }
+__host__ __device__ constexpr int st_ring(int Kp) { return 16 * st_arow(Kp) + 16 * (Kp / 32); }
+__host__ __device__ constexpr int st_lds(int Kp, int nst) { return st_ring(Kp) + 4 * nst * kStBytes; }
+
+template <int NST>
+__global__ __launch_bounds__(256, 1) void lin_stream_kernel(const uint8_t* __restrict__ aq, const uint8_t* __restrict__ as,
+                                                            const uint8_t* __restrict__ wp,
+                                                            const uint8_t* __restrict__ ws, float* __restrict__ y,
+                                                            int M, int N, int Kp, int tiles) {
+    extern __shared__ __align__(16) uint8_t s_dyn[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int cbytes = Kp >> 1, nch = Kp >> 5, nseg = Kp / kStK;
+    const int nw = 4 * gridDim.x, w0 = 4 * blockIdx.x + wave;
+    const int mine = w0 < tiles ? (tiles - w0 + nw - 1) / nw : 0;   // the wave's tiles
+    const int total = mine * nseg;
+    uint8_t* asl = s_dyn + 16 * st_arow(Kp);
+    uint8_t* ring = s_dyn + st_ring(Kp) + wave * (NST * kStBytes);
+    const uint32_t ring_lds = __builtin_amdgcn_readfirstlane(mx::lds_addr(ring));
+    // lane offsets within a stage: data copy j covers rows 2j, 2j + 1 (slot lane % 32
+    // of row lane / 32 holds chunk slot ^ row), the scale copy 16 bytes of row lane / 2
+    uint32_t dvo[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int row = 2 * j + (lane >> 5);
+        dvo[j] = (uint32_t)(row * cbytes + (((lane & 31) ^ row) << 4));
+    }
+    const uint32_t svo = (uint32_t)((lane >> 1) * nch + 16 * (lane & 1));
+    int pt = w0, pseg = 0;                                          // the next stage to copy
+    auto issue = [&](int slot) {
+        const int t = min(pt, tiles - 1);                           // past the wave's last: copied, not used
+        const int64_t n0 = (int64_t)t * 16;
+        const int rows = min(16, N - (int)n0);
+        const mx::v4u rw = mx::buf_rsrc(wp + n0 * cbytes, (int64_t)rows * cbytes);
+        const mx::v4u rs = mx::buf_rsrc(ws + n0 * nch, (int64_t)rows * nch);
+        const uint32_t dst = ring_lds + slot * kStBytes;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mx::dma16(dvo[j], rw, (uint32_t)(pseg * kStRowB), dst + j * 1024);
+        if (lane < 32) mx::dma16(svo, rs, (uint32_t)(pseg * kStNch), dst + kStData);
+        if (++pseg == nseg) {
+            pseg = 0;
+            pt += nw;
+        }
+    };
+    if (total > 0) {
+#pragma unroll
+        for (int s = 0; s < NST - 1; ++s) issue(s);
+    }
+    // the activation rows and their scale codes (zeros and 127 past M)
+    for (int i = tid; i < 16 * nch; i += 256) {
+        const int m = i / nch, c = i - m * nch;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        uint8_t code = 127;
+        if (m < M) {
+            v = *reinterpret_cast<const uint4*>(aq + (int64_t)m * cbytes + 16 * c);
+            code = as[(int64_t)m * nch + c];
+        }
+        *reinterpret_cast<uint4*>(s_dyn + m * st_arow(Kp) + 16 * c) = v;
+        asl[i] = code;
+    }
+    __syncthreads();
+    const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(y, (short)0, (uint32_t)M * (uint32_t)N * 4u, 0x00020000);
+    const uint8_t* arow = s_dyn + r * st_arow(Kp);
+    const uint8_t* asr = asl + r * nch;
+    mx::v4f acc = {0.f, 0.f, 0.f, 0.f};
+    int seg = 0, t = w0, slot = 0;
+    for (int st = 0; st < total; ++st) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * kStCopies) : "memory");
+        const uint8_t* wd = ring + slot * kStBytes;
+        const uint4 b0 = *reinterpret_cast<const uint4*>(wd + kStData + r * kStNch);
+        const uint4 b1 = *reinterpret_cast<const uint4*>(wd + kStData + r * kStNch + 16);
+        const uint4 a0 = *reinterpret_cast<const uint4*>(asr + seg * kStNch);
+        const uint4 a1 = *reinterpret_cast<const uint4*>(asr + seg * kStNch + 16);
+        const uint32_t bw[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+        const uint32_t aw[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        uint4 bv[8], av[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            bv[s] = *reinterpret_cast<const uint4*>(wd + r * kStRowB + (((4 * s + g) ^ r) << 4));
+            av[s] = *reinterpret_cast<const uint4*>(arow + seg * kStRowB + ((4 * s + g) << 4));
+        }
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            acc = mx::mfma16_fp4(av[s], bv[s], acc, (aw[s] >> (8 * g)) & 0xFFu, (bw[s] >> (8 * g)) & 0xFFu);
+        // the stage's reads are done: the copies of the stage NST - 1 ahead may go to the slot before it
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        issue(slot == 0 ? NST - 1 : slot - 1);
+        slot = slot + 1 == NST ? 0 : slot + 1;
+        if (++seg == nseg) {
+            mx::pin(acc);
+            const int col = 16 * t + r;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = 4 * g + i;
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i]), ry,
+                                                      m < M && col < N ? (uint32_t)(m * N + col) * 4u : 0x80000000u, 0, 0);
+            }
+            acc = mx::v4f{0.f, 0.f, 0.f, 0.f};
+            seg = 0;
+            t += nw;
+        }
+    }
+    // the copies past the last stage land before the LDS goes to another workgroup
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // ---------------------------------------------------------------- RMSNorm -> lin_pq
 // The decode step's "x = x + bf16(o); h = rms_norm(x) -> MXFP4; y = lin_pq(h)"
 // (runtime/model_runner_v2.py:185-187 and :208 + :147-152; RMSNorm
@@ -769,10 +899,48 @@ int lin_pq_gemv(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const 
     return MXFP4_OK;
 }
 
+// Stages (row tiles x K / 1024) from which the streaming kernel takes over,
+// four per wave: with fewer its start, the first copies' latency and the
+// activation rows, shows (MI355X, us, tile per wave / streaming: 2048 stages
+// 16384 x 2048 7.3 / 7.3 and 32768 x 1024 6.1 / 7.0, 3000 stages 24000 x 2048
+// 10.4 / 9.3, 4096 stages 16384 x 4096 13.3 / 11.2 and 32768 x 2048 11.3 /
+// 10.8, 18992 stages 151936 x 2048 42.5 / 34.5).  With one stage a tile the
+// ring is drained by half as much work per output, so it takes more of them:
+// 65536 x 1024 is 11.1 / 10.6 with eight rows but 9.4 / 10.1 with one, 98400 x
+// 1024 15.3 / 13.6 and 12.7 / 13.0, 151936 x 1024 17.7 / 17.6 with one.
+constexpr int kStreamStages = 4096, kStreamStages1 = 8192;
+
+template <int NST>
+int launch_lin_stream_n(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y, int M,
+                        int N, int Kp, int tiles, hipStream_t st) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&lin_stream_kernel<NST>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (attr != hipSuccess) {
+        set_error("lin_pq: hipFuncSetAttribute: %s", hipGetErrorString(attr));
+        return (int)attr;
+    }
+    // as many waves as take the same number of tiles each, up to four on each of 256 CUs
+    const int rounds = (tiles + 1023) / 1024;
+    const int waves = (tiles + rounds - 1) / rounds;
+    hipLaunchKernelGGL(lin_stream_kernel<NST>, dim3((unsigned)((waves + 3) / 4)), dim3(256), st_lds(Kp, NST), st, xq, xsc,
+                       wp, wsc, y, M, N, Kp, tiles);
+    return launch_status("lin_pq_stream");
+}
+
+int launch_lin_stream(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y, int M,
+                      int N, int Kp, int tiles, hipStream_t st) {
+    static_assert(st_lds(2048, 4) <= 160 * 1024 && st_lds(4096, 3) <= 160 * 1024, "ring");
+    return Kp <= 2048 ? launch_lin_stream_n<4>(xq, xsc, wp, wsc, y, M, N, Kp, tiles, st)
+                      : launch_lin_stream_n<3>(xq, xsc, wp, wsc, y, M, N, Kp, tiles, st);
+}
+
 int lin_small(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y, int M, int N,
               int Kp, hipStream_t st) {
     const int tiles = (N + 15) / 16;
     const int steps = (Kp / 32 + 3) / 4;
+    if (Kp % kStK == 0 && Kp <= 4096 && N <= (1 << 24) && tiles * (Kp / kStK) >= (Kp > kStK ? kStreamStages : kStreamStages1) &&
+        ((((uintptr_t)xq | (uintptr_t)xsc | (uintptr_t)wp | (uintptr_t)wsc) & 15) == 0))
+        return launch_lin_stream(xq, xsc, wp, wsc, y, M, N, Kp, tiles, st);
     int S = 1;
     while (S < 16 && 2 * S <= steps && (int64_t)tiles * S < 1024) S *= 2;
     const int spw = (steps + S - 1) / S;
