@@ -7,9 +7,10 @@
 //   grids 256 x 256 with 8 waves: a wave owns 128 x 64 as 4 x 2
 //   v_mfma_scale_f32_32x32x64_f8f6f4 accumulators.  (NW = 4, 128 x 128 per
 //   wave with the accumulators in AGPRs, would read a third less from LDS but
-//   does not fit the register file without spills.)  Smaller grids take
-//   128 x 128 or 64 x 64 tiles with 4 waves and a deeper ring (the launcher
-//   picks the instance); every instance runs the same MFMA chain per output.
+//   does not fit the register file without spills.)  The other instances take
+//   at most half of the LDS, so two workgroups share a CU and one's copies,
+//   first latency and stores run under the other's MFMAs (the launcher picks);
+//   every instance runs the same MFMA chain per output.
 // * K step BK (BK/2 bytes of each operand row; BK = 256 here).  Global -> LDS
 //   with buffer_load_dwordx4 ... lds (no registers, no repacking): lane i of an
 //   instruction writes LDS bytes [16i, 16i+16) of a 1 KB block of whole rows.
@@ -17,7 +18,7 @@
 //   an XOR swizzle, chosen so that the 16 lanes of one ds_read_b128 phase
 //   (16 consecutive rows, one chunk each, 256 bytes over the 64 banks) hit 16
 //   different 16-byte bank groups.
-// * NSTAGE stages in a ring, one workgroup per CU: the copies of the next
+// * NSTAGE stages in a ring: the copies of the next
 //   NSTAGE-1 steps are in flight during the MFMAs of a step.  A step's copies
 //   are spread over its four MFMA substeps (issued in one burst they held
 //   back each wave's MFMAs while the memory pipeline accepted them).  Every
@@ -173,7 +174,8 @@ __device__ __forceinline__ CopyState copy_state(const G2Args& g, int m0, int n0)
 template <int BM, int BN, int BK, int NW, bool RG>
 __device__ __forceinline__ void issue_part(const G2Args& g, const CopyState& c, uint32_t buf, int k0, int part) {
     using T = Tile<BM, BN, BK, NW, RG>;
-    static_assert(T::A_CP % 2 == 0 && T::W_CP % 2 == 0, "even copy counts (swizzle key parity)");
+    static_assert((T::A_CP % 2 == 0 || T::A_CP == 1) && (T::W_CP % 2 == 0 || T::W_CP == 1),
+                  "even copy counts, or one (swizzle key parity)");
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: scalar selects below
     const uint32_t cbytes = g.Kp >> 1, nch = g.Kp >> 5;
     // RG: past the row's last block, an offset out of every range (zeros)
@@ -309,7 +311,8 @@ __device__ __forceinline__ void mfma_step(const uint8_t* cur, mx::v16f (&acc)[Ti
 }
 
 template <int BM, int BN, int BK, int NSTAGE, int NW, bool RG>
-__global__ __launch_bounds__(64 * NW, 1) void gemm2_kernel(G2Args g) {
+__global__ __launch_bounds__(64 * NW, (2 * NSTAGE * Tile<BM, BN, BK, NW, RG>::STAGE > 160 * 1024 ? 1 : 2) * NW / 4) void
+gemm2_kernel(G2Args g) {
     using T = Tile<BM, BN, BK, NW, RG>;
     constexpr int TN = T::TN;
     static_assert(NSTAGE >= 2 && NSTAGE * T::STAGE <= 160 * 1024, "LDS ring");
@@ -376,10 +379,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm2_kernel(G2Args g) {
 #pragma unroll
     for (int i = 0; i < T::IM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            if constexpr (NW == 4) mx::pin_acc(acc[i][j]);
-            else mx::pin(acc[i][j]);
-        }
+        for (int j = 0; j < TN; ++j) mx::pin(acc[i][j]);
     // accumulator element e of lane l: row 8*(e/4) + 4*(l/32) + e%4, column l%32;
     // non-temporal stores (y is not read back by this launch; measured:
     // 2048 x 2048 x 768 9.2 -> 7.9 us)
@@ -436,21 +436,34 @@ int launch_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const
 template <bool RG>
 int pick_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y, int M, int N,
                int Kp, hipStream_t st) {
-    // Tile by grid size: 256 x 256 (2 stages) when it gives at least 128
-    // tiles; else 128 x 128 (4 stages) when that gives at least 192; else
-    // 64 x 64 with 8 stages, i.e. up to 7 K-steps of copies in flight, so a
-    // small grid pays about one memory latency instead of one per K-step --
-    // or with 4 stages (two workgroups per CU) when one per CU would take
-    // two rounds.  Measured on MI355X: 512 x 1536 x 2048 in 6.5 us against
-    // 11.1 us for 128 x 128 tiles; all tiles give the same bits (the same
-    // MFMA chain per output).
+    // The tile by the number of tiles a grid gives (MI355X, us):
+    //  * at most 256 of 64 x 64 (one a CU): 64 x 64, four stages.  512 x 2048 x
+    //    2048 5.9, 32 x 2048 x 4096 7.3; 64 x 128 7.6 and 9.8; eight stages
+    //    (one workgroup per CU, whatever the grid) 6.9 and 8.3.
+    //  * K of 1536 on and at least 160 of 256 x 256, unless half of each would be
+    //    padding (t128 = 2 t256): 4096^2 x 2048 28.8 against 31.2 with 128 x 128,
+    //    2048 x 5120 x 2048 21.6 against 23.7; but 144 tiles 30.9 against 29.7,
+    //    128 tiles 20.0 against 17.5, and with less K to each output's store
+    //    4096^2 x 768 20.0 against 18.4.
+    //  * at least 160 of 128 x 128 and M > 64: 128 x 128.  1500 x 3000 x 1024
+    //    10.8 against 12.8 with 64 x 128 (15.5 with four waves and four stages, one
+    //    workgroup per CU); at 512 x 5120 x 2048, 160 tiles, 9.9 against 11.4.
+    //    With K < 1024 the smaller tile goes on a little longer: 2048 x 3000 x 768
+    //    10.7 against 11.5, 4096^2 x 768 21.0 against 18.4.
+    //  * else 64 x 128, three stages (two with ragged scales, to stay at two
+    //    workgroups per CU): 1000 x 2000 x 2048 7.8 against 8.6 with 64 x 64, 32 x
+    //    151936 x 2048 40.2 against 45.2 and 62 with 256 x 256.
+    // All tiles give the same bits (the same MFMA chain per output).
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    const int64_t t64x128 = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
     const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-    if (t256 >= 128) return launch_gemm2<256, 256, 256, 2, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
-    if (t128 >= 192) return launch_gemm2<128, 128, 256, 4, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
-    if (t64 > 256) return launch_gemm2<64, 64, 256, 4, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
-    return launch_gemm2<64, 64, 256, 8, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    if (t64 <= 256) return launch_gemm2<64, 64, 256, 4, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    if (Kp >= 1536 && t256 >= 160 && 2 * t128 >= 5 * t256)
+        return launch_gemm2<256, 256, 256, 2, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    if (M > 64 && t128 >= 160 && !(Kp < 1024 && t64x128 <= 768))
+        return launch_gemm2<128, 128, 256, 2, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    return launch_gemm2<64, 128, 256, RG ? 2 : 3, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
 }
 
 int lin_pq_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y,

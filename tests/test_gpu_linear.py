@@ -58,9 +58,17 @@ FWD_SHAPES = [(16, 8, 64), (16, 8, 100), (16, 8, 40), (1, 8, 64), (1, 32, 64), (
 
 
 # M > 16 with Kp % 256 != 0: one block and one short of a step, scale rows that start at any byte of a dword,
-# a tail after full steps on each tile size (64 x 64 in eight and four stages, 128 x 128, 256 x 256)
+# a tail after full steps on each tile size (64 x 64; 64 x 128 from (1100, 900) on; 128 x 128 and 256 x 256 the last two)
 RAGGED_SHAPES = [(17, 33, 32), (65, 127, 224), (333, 1000, 2080), (100, 129, 1312 + 256), (200, 64, 2048 + 96),
-                 (1100, 900, 544), (1500, 2100, 800), (3000, 3100, 288)]
+                 (1100, 900, 544), (1500, 2100, 800), (3000, 3100, 288), (2600, 4100, 1568)]
+
+
+# the tile rule's other sides: M up to one and just past one 64- and 128-row tile with many columns, 144 and 160 tiles of
+# 256 x 256, K on both sides of 1024 and 1536
+@pytest.mark.parametrize("M,N,K", [(64, 5000, 512), (65, 10300, 512), (129, 5300, 1024), (2300, 4000, 1536), (2500, 4090, 1536),
+                                   (2300, 2500, 1280), (520, 5121, 2048)])
+def test_lin_pq_tile_rule_vs_oracle(dext, M, N, K):
+    test_lin_pq_vs_oracle(dext, M, N, K)
 
 
 @pytest.mark.parametrize("M,N,K", RAGGED_SHAPES)
