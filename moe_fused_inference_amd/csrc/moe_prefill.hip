@@ -17,13 +17,13 @@
 //   2. quantize_rows      h (T, H) bf16 -> fp16-rounded -> MXFP4, once per
 //                         token (the per-row quantization does not depend on
 //                         which expert gathers the row).
-//   3. grouped GEMM, gate/up   workgroup (feature tile, expert): for every
-//                         128-token tile of the expert, A = gathered token
-//                         rows, W = 64 gate rows + the same 64 up rows; the
+//   3. grouped GEMM, gate/up   tiles of (expert, up to 192 of its tokens, 128
+//                         features): A = gathered token rows, W = the gate
+//                         rows of the features + their up rows; the
 //                         epilogue computes h = silu(g)*u in fp32, rounds it
 //                         to fp16 (the x.to(half) of the `forward` binding)
 //                         and quantizes it to MXFP4 in registers.
-//   4. grouped GEMM, down      workgroup (output tile, expert): A = the
+//   4. grouped GEMM, down      tiles of 256 output columns: A = the
 //                         expert's quantized h rows; the epilogue writes
 //                         bf16(bf16(y) * score) per (token, slot) pair.
 //   5. combine_kernel     out[t] = bf16(sum over the token's slots, fp32,
@@ -31,12 +31,11 @@
 //                         nothing, as an id missing from `experts` does in
 //                         the reference.
 //
-// MFMA tiling is that of the lin_pq GEMM (128x128 tiles, K step 256, LDS
-// double buffer, v_mfma_scale_f32_32x32x64_f8f6f4), with the operands
+// The grouped GEMMs use v_mfma_scale_f32_32x32x64_f8f6f4 with the operands
 // swapped: the weight tile is the MFMA's A operand, so each lane ends with
 // one token and 16 features of a 32-feature block.  The 32-block amax of h is
 // then one exchange with lane l^32, and the nibbles pack into 8-byte stores.
-#include <type_traits>
+#include <algorithm>
 
 #include "lds_dma.h"
 #include "mx_device.h"
@@ -50,12 +49,6 @@ int quantize_rows_impl(const void* x, int src_dtype, int round_to_f16, int64_t l
 
 namespace {
 
-constexpr int BM = 128, BN = 128, BK = 256;   // tokens, weight rows, K per step
-constexpr int ROWB = BK / 2;
-constexpr int LDSROW = ROWB + 16;
-constexpr int SCB = BK / 32;
-constexpr int TILE_BYTES = BM * LDSROW;
-constexpr int BUF_BYTES = 2 * TILE_BYTES + 2 * BM * SCB;
 constexpr int kMaxExperts = 1024;
 constexpr int kMaxTopk = 32;
 
@@ -219,10 +212,10 @@ __device__ __forceinline__ int id_bits(int n_exp) { return 32 - __clz(max(n_exp 
 // routing, and the count's few latency-bound workgroups leave the CUs free.
 struct XQuant {
     const void* x;      // (T, H) bf16
-    int T, H;
+    int T, H, Kp;       // Kp: H padded to whole K steps
     int lt, gx;         // quantize_rows_kernel's layout: 2^lt threads per row, gx row groups
-    uint8_t* q;         // (T, H/2)
-    uint8_t* s;         // (T, H/32)
+    uint8_t* q;         // (T, Kp/2)
+    uint8_t* s;         // (T, Kp/32)
 };
 
 __global__ __launch_bounds__(64 * kRtWaves) void route_count_kernel(const int64_t* __restrict__ topi, int P, int n_exp,
@@ -235,7 +228,7 @@ __global__ __launch_bounds__(64 * kRtWaves) void route_count_kernel(const int64_
         const int bx = local % xq.gx, by = local / xq.gx;
         const int64_t row = (int64_t)bx * (256 >> xq.lt) + (tid >> xq.lt);
         const int u = by * (1 << xq.lt) + (tid & ((1 << xq.lt) - 1));
-        mxq::quantize_unit<MXFP4_DT_BF16, 1>(xq.x, xq.H, xq.T, xq.H, xq.H, true, row, u, xq.q, xq.s);
+        mxq::quantize_unit<MXFP4_DT_BF16, 1>(xq.x, xq.H, xq.T, xq.H, xq.Kp, true, row, u, xq.q, xq.s);
         return;
     }
     if (qctr && blockIdx.x == 0 && tid < 16) qctr[tid] = 0;   // the grouped GEMMs' tile queues (8 each)
@@ -377,78 +370,29 @@ struct TableW {                  // device table (n_experts, 6) int64: gate wp/w
 };
 
 struct GArgs {
-    const uint8_t* aq;       // GATEUP: token rows (T, H/2); DOWN: sorted h rows (P, Mi/2)
+    const uint8_t* aq;       // GATEUP: token rows (T); DOWN: sorted h rows (P)
     const uint8_t* as;       // matching scale rows
+    int ald, asld;           // bytes from row to row of aq / as (whole K steps)
     const int* counts;
     const int* offs;
     const int* pairs;
     int topk;
     int Kp;                  // K of this GEMM: H (gate/up) or Mi (down)
     int Nw;                  // weight rows per projection: Mi (gate/up) or H (down)
-    uint8_t* hq;             // GATEUP out: (P, Mi/2) MXFP4 h in sorted order
-    uint8_t* hs;             //             (P, Mi/32)
+    uint8_t* hq;             // GATEUP out: MXFP4 h in sorted order, rows hld bytes apart
+    uint8_t* hs;             //             and its scales, hsld apart
+    int hld, hsld;
     uint16_t* yd;            // DOWN out: (P, H) bf16 at the pair's own index
     const float* sscore;     // DOWN: (P) routing weights in sorted pair order
     int a_rows;              // rows of aq / as (T for gate/up, P for down)
 };
 
-struct StageRegs {
-    uint4 a[4];
-    uint4 w[4];
-    uint2 sc;
-};
-
-// One K step: 4 x 16 B of A rows and of W rows per thread, 8 scale bytes of
-// one row (threads 0..127: A row, 128..255: W row).  Row base pointers are
-// resolved once per token tile (gathered tokens, gate/up interleave).
-__device__ __forceinline__ void load_stage(StageRegs& r, const uint8_t* const arow[4], const uint8_t* const wrow[4],
-                                           const uint8_t* srow, int Kp, int k0) {
-    const int tid = threadIdx.x;
-    const int nch = Kp >> 5;
-    const int kb0 = k0 >> 5;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int ch = tid & 7;
-        const bool kok = kb0 + ch < nch;
-        const int off = (k0 >> 1) + ch * 16;
-        r.a[i] = kok ? *reinterpret_cast<const uint4*>(arow[i] + off) : make_uint4(0, 0, 0, 0);
-        r.w[i] = kok ? *reinterpret_cast<const uint4*>(wrow[i] + off) : make_uint4(0, 0, 0, 0);
-    }
-    const uint8_t* sp = srow + kb0;
-    if (kb0 + SCB <= nch && (((uintptr_t)sp) & 7) == 0) {
-        r.sc = *reinterpret_cast<const uint2*>(sp);
-    } else {
-        uint32_t lo = 0, hi = 0;
-#pragma unroll
-        for (int j = 0; j < SCB; ++j) {
-            const uint32_t b = (kb0 + j < nch) ? (uint32_t)sp[j] : 127u;
-            if (j < 4) lo |= b << (8 * j);
-            else hi |= b << (8 * (j - 4));
-        }
-        r.sc = make_uint2(lo, hi);
-    }
-}
-
-__device__ __forceinline__ void store_stage(const StageRegs& r, uint8_t* buf) {
-    const int tid = threadIdx.x;
-    uint8_t* la = buf;
-    uint8_t* lw = buf + TILE_BYTES;
-    uint8_t* lsa = buf + 2 * TILE_BYTES;
-    uint8_t* lsw = lsa + BM * SCB;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = (tid >> 3) + 32 * i;
-        const int ch = tid & 7;
-        *reinterpret_cast<uint4*>(la + row * LDSROW + ch * 16) = r.a[i];
-        *reinterpret_cast<uint4*>(lw + row * LDSROW + ch * 16) = r.w[i];
-    }
-    const int row = tid & 127;
-    *reinterpret_cast<uint2*>((tid >= 128 ? lsw : lsa) + row * SCB) = r.sc;
-}
-
-__device__ __forceinline__ uint32_t scale_word(const uint8_t* srow, int h) {
-    const uint2 v = *reinterpret_cast<const uint2*>(srow);
-    return __builtin_amdgcn_perm(v.y, v.x, h ? 0x07050301u : 0x06040200u);
+// Scale word of a lane: byte ks = block 2*ks + h of the step's eight bytes lo,
+// hi; RG: the bytes outside `keep` (blocks past the row) become 127.
+template <bool RG>
+__device__ __forceinline__ uint32_t scale_word(uint32_t lo, uint32_t hi, int h, uint32_t keep) {
+    const uint32_t w = __builtin_amdgcn_perm(hi, lo, h ? 0x07050301u : 0x06040200u);
+    return RG ? (w & keep) | (0x7F7F7F7Fu & ~keep) : w;
 }
 
 template <int OP>
@@ -472,35 +416,19 @@ __device__ __forceinline__ int weight_row(int rho, int n0, int& proj) {
     return n0 + rho;
 }
 
-// Down epilogue inputs of the lane's two token rows rbase + 32i + lr: the
-// pair index and its routing weight (loaded ahead of the K loop by the
-// kernels that can, so the epilogue waits on no load).
-__device__ __forceinline__ void down_rows(const GArgs& g, int off, int mt, int mrows, int rbase, int lr, int (&pp)[2],
-                                          float (&ss)[2]) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int rloc = rbase + 32 * i + lr;
-        pp[i] = rloc < mrows ? g.pairs[off + mt + rloc] : 0;
-        ss[i] = rloc < mrows ? g.sscore[off + mt + rloc] : 0.0f;
-    }
-}
-
-// Epilogue of a 128 x 128 tile (acc[i][j] of the 2 x 2 wave layout):
-// gate/up -> h = silu(g)*u, fp16, MXFP4 rows in sorted pair order; down ->
-// bf16(bf16(y) * score) at the pair's own index (pp / ss from down_rows).
-// NI: how many of the two token blocks to process (1: only acc[0]).
-template <int MODE, int NI = 2>
-__device__ __forceinline__ void tile_epilogue(mx::v16f (&acc)[2][2], const GArgs& g, int n0, int off, int mt,
-                                              int mrows, int rbase, int wn, int lr, int h, const int (&pp)[2],
-                                              const float (&ss)[2], int istride = 32) {
-    // acc[i][j] element q of lane l: token rbase + istride*i + l%32, weight
-    // row wn*64 + 32j + 8(q/4) + 4h + q%4 of the tile
-    if (MODE == MODE_GATEUP) {
+// Gate/up epilogue of NI 32-token blocks of a wave, 64 tile rows apart: h =
+// silu(g)*u, fp16, MXFP4 rows in sorted pair order.
+template <int NI>
+__device__ __forceinline__ void gateup_epilogue(mx::v16f (&acc)[2][2], const GArgs& g, int n0, int off, int mt,
+                                                int mrows, int rbase, int wn, int lr, int h) {
+    // acc[i][j] element q of lane l: token rbase + 64*i + l%32, weight row
+    // wn*64 + 32j + 8(q/4) + 4h + q%4 of the tile
+    {
         const int fb = n0 + 32 * wn;           // first feature of this wave's 32-block
         const int Mi = g.Nw;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-            const int rloc = rbase + istride * i + lr;
+            const int rloc = rbase + 64 * i + lr;
             float v[16];
             float amax = 0.0f;
 #pragma unroll
@@ -530,318 +458,10 @@ __device__ __forceinline__ void tile_epilogue(mx::v16f (&acc)[2][2], const GArgs
             }
             if (rloc < mrows && fb < Mi) {
                 const int64_t srow_i = off + mt + rloc;
-                *reinterpret_cast<uint2*>(g.hq + srow_i * (Mi >> 1) + (fb >> 1) + 8 * h) = d;
-                if (h == 0) g.hs[srow_i * (Mi >> 5) + (fb >> 5)] = (uint8_t)code;
+                *reinterpret_cast<uint2*>(g.hq + srow_i * g.hld + (fb >> 1) + 8 * h) = d;
+                if (h == 0) g.hs[srow_i * g.hsld + (fb >> 5)] = (uint8_t)code;
             }
         }
-    } else {
-        const int H = g.Nw;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int rloc = rbase + istride * i + lr;
-            if (rloc < mrows) {
-                const int p = pp[i];
-                const float sc = ss[i];
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int cb = n0 + wn * 64 + 32 * j;   // 32-column block
-                    if (cb < H) {
-#pragma unroll
-                        for (int q4 = 0; q4 < 4; ++q4) {
-                            uint32_t b[2];
-#pragma unroll
-                            for (int r = 0; r < 2; ++r) {
-                                // bf16(bf16(y) * score), two at a time
-                                const uint32_t y2 = mx::f32x2_to_bf16x2(acc[i][j][4 * q4 + 2 * r], acc[i][j][4 * q4 + 2 * r + 1]);
-                                b[r] = mx::f32x2_to_bf16x2(__uint_as_float(y2 << 16) * sc,
-                                                           __uint_as_float(y2 & 0xFFFF0000u) * sc);
-                            }
-                            *reinterpret_cast<uint2*>(g.yd + (int64_t)p * H + cb + 8 * q4 + 4 * h) = make_uint2(b[0], b[1]);
-                        }
-                    }
-                }
-            }
-        }
-    }
-}
-
-template <int MODE, class W>
-__global__ __launch_bounds__(256, 2) void grouped_gemm_kernel(GArgs g, W w) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    const int e = blockIdx.y;
-    const int cnt = g.counts[e];
-    if (cnt == 0) return;
-    const int off = g.offs[e];
-    // gate/up: 64 features per workgroup; down: 128 output columns
-    const int n0 = blockIdx.x * (MODE == MODE_GATEUP ? BN / 2 : BN);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lr = lane & 31;
-    const int h = lane >> 5;
-    const int cbytes = g.Kp >> 1;
-    const int nch = g.Kp >> 5;
-    const int nsteps = (g.Kp + BK - 1) / BK;
-
-    // weight rows of this thread (fixed for the whole workgroup)
-    const uint8_t* wrow[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        int proj;
-        const int rr = min(weight_row<MODE>((tid >> 3) + 32 * i, n0, proj), g.Nw - 1);
-        wrow[i] = w.p(e, proj) + (int64_t)rr * cbytes;
-    }
-    const uint8_t* wsrow;
-    {
-        int proj;
-        const int rr = min(weight_row<MODE>(tid & 127, n0, proj), g.Nw - 1);
-        wsrow = w.s(e, proj) + (int64_t)rr * nch;
-    }
-
-    for (int mt = 0; mt < cnt; mt += BM) {
-        const int mrows = min(BM, cnt - mt);
-        // token (A) rows of this thread, clamped to the tile's last valid row
-        const uint8_t* arow[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = min((tid >> 3) + 32 * i, mrows - 1);
-            const int src = MODE == MODE_GATEUP ? g.pairs[off + mt + r] / g.topk : off + mt + r;
-            arow[i] = g.aq + (int64_t)src * cbytes;
-        }
-        const uint8_t* srow = wsrow;
-        if (tid < 128) {
-            const int r = min(tid, mrows - 1);
-            const int src = MODE == MODE_GATEUP ? g.pairs[off + mt + r] / g.topk : off + mt + r;
-            srow = g.as + (int64_t)src * nch;
-        }
-
-        mx::v16f acc[2][2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
-
-        StageRegs st;
-        load_stage(st, arow, wrow, srow, g.Kp, 0);
-        store_stage(st, smem);
-        __syncthreads();
-        for (int it = 0; it < nsteps; ++it) {
-            uint8_t* cur = smem + (it & 1) * BUF_BYTES;
-            const bool more = it + 1 < nsteps;
-            if (more) load_stage(st, arow, wrow, srow, g.Kp, (it + 1) * BK);
-            const uint8_t* la = cur;
-            const uint8_t* lw = cur + TILE_BYTES;
-            const uint8_t* lsa = cur + 2 * TILE_BYTES;
-            const uint8_t* lsw = lsa + BM * SCB;
-            uint32_t sa[2], sb[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                sa[i] = scale_word(lsa + (wm * 64 + i * 32 + lr) * SCB, h);
-                sb[i] = scale_word(lsw + (wn * 64 + i * 32 + lr) * SCB, h);
-            }
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                uint4 af[2], bf[2];
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    af[i] = *reinterpret_cast<const uint4*>(la + (wm * 64 + i * 32 + lr) * LDSROW + ks * 32 + h * 16);
-                    bf[i] = *reinterpret_cast<const uint4*>(lw + (wn * 64 + i * 32 + lr) * LDSROW + ks * 32 + h * 16);
-                }
-                // D[weight row][token]: the weight tile is the MFMA A operand
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        if (ks == 0) acc[i][j] = mfma32<0>(bf[j], af[i], acc[i][j], sb[j], sa[i]);
-                        if (ks == 1) acc[i][j] = mfma32<1>(bf[j], af[i], acc[i][j], sb[j], sa[i]);
-                        if (ks == 2) acc[i][j] = mfma32<2>(bf[j], af[i], acc[i][j], sb[j], sa[i]);
-                        if (ks == 3) acc[i][j] = mfma32<3>(bf[j], af[i], acc[i][j], sb[j], sa[i]);
-                    }
-            }
-            if (more) store_stage(st, smem + ((it + 1) & 1) * BUF_BYTES);
-            __syncthreads();
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) mx::pin(acc[i][j]);
-
-        int pp[2] = {0, 0};
-        float ss[2] = {0.0f, 0.0f};
-        if (MODE == MODE_DOWN) down_rows(g, off, mt, mrows, wm * 64, lr, pp, ss);
-        tile_epilogue<MODE>(acc, g, n0, off, mt, mrows, wm * 64, wn, lr, h, pp, ss);
-        __syncthreads();   // LDS buffers are refilled by the next token tile
-    }
-}
-
-// ------------------------------------------------------------------ LDS-copy ring variant
-// Tiles of 256 tokens x 128 weight rows (a wave: 128 tokens x 64 rows), so an
-// expert's ~128-250 routed tokens take one pass over its weights: with
-// 128-token tiles half of the experts streamed their weights twice, the
-// second time for a handful of tokens.  The operands are copied global ->
-// LDS by buffer_load ... lds (no registers) into a ring of D_NST stages of
-// 128-wide K slices, two slices of copies in flight while a third is
-// multiplied.  LDS rows are 64 bytes with an XOR swizzle of their four
-// 16-byte chunks, so the 16 lanes of an operand read hit distinct bank
-// groups.  The epilogues are the 128 x 128 kernel's.  Requires Kp % 128 == 0.
-constexpr int DM = 256;                     // tokens per tile
-constexpr int DK = 128;                     // K per stage
-constexpr int DROWB = DK / 2;               // bytes per row per stage
-constexpr int D_A = DM * DROWB;             // 16 KB of token rows
-constexpr int D_W = BN * DROWB;             // 8 KB of weight rows
-constexpr int D_SA = DM * 4;                // 4 scale bytes per row
-constexpr int D_SW = BN * 4;
-constexpr int D_STAGE = D_A + D_W + D_SA + D_SW;
-constexpr int D_NST = 3;
-constexpr int D_COPIES = 8;                 // per wave per stage: 4 token-row, 2 weight-row, 2 scale copies
-
-__device__ __forceinline__ int dswz(int r) { return ((r >> 1) ^ (r >> 2)) & 3; }
-
-__device__ __forceinline__ uint32_t scale4(const uint8_t* p, int h) {
-    const uint32_t v = *reinterpret_cast<const uint32_t*>(p);
-    return __builtin_amdgcn_perm(v, v, h ? 0x0C0C0301u : 0x0C0C0200u);   // byte ks = block 2ks + h
-}
-
-template <int MODE, class W>
-__global__ __launch_bounds__(256, 2) void grouped_gemm_dma_kernel(GArgs g, W w) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    const int e = blockIdx.y;
-    const int cnt = g.counts[e];
-    if (cnt == 0) return;
-    const int off = g.offs[e];
-    const int n0 = blockIdx.x * (MODE == MODE_GATEUP ? BN / 2 : BN);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lr = lane & 31;
-    const int h = lane >> 5;
-    const uint32_t cbytes = (uint32_t)g.Kp >> 1, nch = (uint32_t)g.Kp >> 5;
-    const int nsteps = g.Kp / DK;
-    const uint32_t ring = __builtin_amdgcn_readfirstlane(mx::lds_addr(smem));
-    const int slot = lane & 3;
-
-    // weight-row copies: 1 KB blocks 2*wave, 2*wave+1 of the W tile (16 rows
-    // each, all of one projection: projections change every 32 rows)
-    mx::v4u wrs[2];
-    uint32_t wvo[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int rho = 16 * (2 * wave + j) + (lane >> 2);
-        int proj;
-        const int rr = min(weight_row<MODE>(rho, n0, proj), g.Nw - 1);
-        wrs[j] = mx::buf_rsrc(w.p(e, proj), (int64_t)g.Nw * cbytes);
-        wvo[j] = (uint32_t)rr * cbytes + ((slot ^ dswz(rho)) << 4);
-    }
-    // scale copies: wave w copies the token rows' scales of rows 64w..64w+63
-    // and (lanes 0..31) the weight rows' of rows 32w..32w+31, one projection
-    uint32_t svo_w;
-    int wproj;
-    {
-        const int rr = min(weight_row<MODE>(32 * wave + (lane & 31), n0, wproj), g.Nw - 1);
-        svo_w = (uint32_t)rr * nch;
-    }
-    const mx::v4u srs_w = mx::buf_rsrc(w.s(e, wproj), (int64_t)g.Nw * nch);
-    const mx::v4u ars = mx::buf_rsrc(g.aq, (int64_t)g.a_rows * cbytes);
-    const mx::v4u asrs = mx::buf_rsrc(g.as, (int64_t)g.a_rows * nch);
-
-    for (int mt = 0; mt < cnt; mt += DM) {
-        const int mrows = min(DM, cnt - mt);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the previous tile's stores
-        uint32_t avo[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int ra = 16 * (4 * wave + j) + (lane >> 2);
-            const int r = min(ra, mrows - 1);
-            const int src = MODE == MODE_GATEUP ? g.pairs[off + mt + r] / g.topk : off + mt + r;
-            avo[j] = (uint32_t)src * cbytes + ((slot ^ dswz(ra)) << 4);
-        }
-        uint32_t svo_a;
-        {
-            const int r = min(64 * wave + lane, mrows - 1);
-            const int src = MODE == MODE_GATEUP ? g.pairs[off + mt + r] / g.topk : off + mt + r;
-            svo_a = (uint32_t)src * nch;
-        }
-
-        auto issue = [&](int stg, int k) {
-            const uint32_t buf = ring + stg * D_STAGE;
-            const uint32_t kofs = (uint32_t)k * DROWB;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) mx::dma16(avo[j], ars, kofs, buf + (4 * wave + j) * 1024);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) mx::dma16(wvo[j], wrs[j], kofs, buf + D_A + (2 * wave + j) * 1024);
-            const uint32_t ksc = (uint32_t)k * 4;
-            mx::dma4(svo_a, asrs, ksc, buf + D_A + D_W + 256 * wave);
-            if (lane < 32) mx::dma4(svo_w, srs_w, ksc, buf + D_A + D_W + D_SA + 128 * wave);
-        };
-
-        mx::v16f acc[4][2];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
-
-#pragma unroll
-        for (int st = 0; st < D_NST - 1; ++st) issue(st, min(st, nsteps - 1));
-        const int key = dswz(lr);
-        for (int it = 0; it < nsteps; ++it) {
-            // this wave's copies of step it have landed (later steps' may still
-            // be in flight) and its reads of step it-1 are done; after the
-            // barrier every wave's.  Past the last step the copies re-read the
-            // last slice, so every step has the same count outstanding.
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((D_NST - 2) * D_COPIES) : "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            issue((it + D_NST - 1) % D_NST, min(it + D_NST - 1, nsteps - 1));
-            const uint8_t* cur = smem + (it % D_NST) * D_STAGE;
-            const uint8_t* la = cur;
-            const uint8_t* lw = cur + D_A;
-            const uint8_t* lsa = cur + D_A + D_W;
-            const uint8_t* lsw = lsa + D_SA;
-            uint32_t sa[4], sb[2];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sa[i] = scale4(lsa + (wm * 128 + i * 32 + lr) * 4, h);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) sb[j] = scale4(lsw + (wn * 64 + j * 32 + lr) * 4, h);
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                const int koff = ((2 * ks + h) ^ key) << 4;
-                uint4 af[4], bf[2];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    af[i] = *reinterpret_cast<const uint4*>(la + (wm * 128 + i * 32 + lr) * DROWB + koff);
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    bf[j] = *reinterpret_cast<const uint4*>(lw + (wn * 64 + j * 32 + lr) * DROWB + koff);
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        if (ks == 0) acc[i][j] = mfma32<0>(bf[j], af[i], acc[i][j], sb[j], sa[i]);
-                        if (ks == 1) acc[i][j] = mfma32<1>(bf[j], af[i], acc[i][j], sb[j], sa[i]);
-                    }
-            }
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the copies issued past the last step
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) mx::pin(acc[i][j]);
-        // the wave's 128 token rows as two 64-row halves of the 128 x 128 epilogue
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            mx::v16f sub[2][2] = {{acc[2 * half][0], acc[2 * half][1]}, {acc[2 * half + 1][0], acc[2 * half + 1][1]}};
-            int pp[2] = {0, 0};
-            float ss[2] = {0.0f, 0.0f};
-            if (MODE == MODE_DOWN) down_rows(g, off, mt, mrows, wm * 128 + 64 * half, lr, pp, ss);
-            tile_epilogue<MODE>(sub, g, n0, off, mt, mrows, wm * 128 + 64 * half, wn, lr, h, pp, ss);
-        }
-        __syncthreads();   // the ring is refilled by the next token tile
     }
 }
 
@@ -866,26 +486,56 @@ __global__ __launch_bounds__(256, 2) void grouped_gemm_dma_kernel(GArgs g, W w) 
 //  * All tiles of one expert run on workgroups of one residue mod 8, i.e.
 //    on one XCD (workgroups are dealt to the 8 XCDs round-robin), so the
 //    expert's gathered token rows are fetched into one L2.
-// Requires Kp % 256 == 0.
+//  * Kp not a multiple of 256 (RG): the token and h rows are the launch's own,
+//    so they sit whole K steps apart; of the weights, which the caller laid
+//    out, the lanes whose chunk lies past a row's end copy zeros, and a row's
+//    scale bytes, which then start at any byte, come as the three aligned dwords
+//    that hold a step's eight and are shifted into place by the reader.  The
+//    blocks past the end read as zeros with scale 127 on both sides.  Measured on
+//    MI355X, 2000 tokens, 60 experts, H = 2016, Mi = 992: 302 us on the
+//    register-staged 128 x 128 tiles these sizes had, 154 us here; 20 tokens, 100
+//    experts, H = 1984, Mi = 736: 104 and 70 us.
 constexpr int X_BM = 192, X_BN = 256;
 constexpr int X_ROWB = 128;                           // bytes per row per K step
 constexpr int X_A = X_BM * X_ROWB;                    // 24 KB of token rows
 constexpr int X_W = X_BN * X_ROWB;                    // 32 KB of weight rows
 constexpr int X_AST = X_A + X_BM * 8;                 // token stage: rows + 8 scale bytes per row
-constexpr int X_WST = X_W + X_BN * 8;                 // weight stage
-constexpr int X_ARING = 3 * X_WST;                    // the token ring follows the 3-stage weight ring
 constexpr int X_THREADS = 512;
-constexpr int X_PP = X_ARING + 2 * X_AST;             // the down tile's pair indices and weights
-constexpr int X_LDS = X_PP + 8 * X_BM;
-static_assert(X_LDS <= 160 * 1024, "x8 LDS layout");
+constexpr int XP_MAXJ = kMaxExperts / 8;              // experts per group
+constexpr int XP_TROW = 136;                          // down transpose: 128 B + 8 per row
+
+// LDS layout: the 3-stage weight ring, the token ring, the down tile's pair
+// indices and weights, the group's units, expert counts and offsets, the
+// queue's unit.
+template <bool RG>
+struct XL {
+    static constexpr int WST = X_W + X_BN * (RG ? 12 : 8);   // weight stage: rows + scale bytes per row
+    static constexpr int ARING = 3 * WST;
+    static constexpr int PP = ARING + 2 * X_AST;
+    static constexpr int UCUM = PP + 8 * X_BM;               // int[XP_MAXJ + 1]: units of the experts below j
+    static constexpr int ECNT = UCUM + 4 * (XP_MAXJ + 1);    // int[XP_MAXJ]: expert counts
+    static constexpr int EOFF = ECNT + 4 * XP_MAXJ;          // int[XP_MAXJ]: expert offsets
+    static constexpr int SLOT = EOFF + 4 * XP_MAXJ;          // int: the unit the queue handed out
+    static constexpr int BYTES = SLOT + 16;
+    static constexpr int WCP = RG ? 6 : 5;                   // weight copies per wave and step
+    static_assert(BYTES <= 160 * 1024 && XP_MAXJ <= 128, "xp LDS layout (two experts per lane in the prefix)");
+    static_assert(8 * 32 * XP_TROW <= WST, "the down transposes fit weight stage 0");
+};
 
 // Per-tile copy plan of one wave: na token-row blocks (8 rows of 128 bytes
 // each), 4 weight-row blocks, one weight-scale copy (32 rows x 8 bytes) and,
 // for waves < 2 na, one token-scale copy.
-struct XCopies {
+struct XCopiesAll {
     mx::v4u ars, wrs, sars, swrs;
     uint32_t avo[3], wvo[4], savo, swvo;
     int na;
+};
+template <bool RG>
+struct XCopies : XCopiesAll {};
+template <>
+struct XCopies<true> : XCopiesAll {
+    uint32_t swvo2;   // the third scale dword's offset, lanes 0 .. 31: row 32 * wave + lane
+    uint32_t shw;     // the shifts of the lane's two operand rows' scales (bits 0-1, 8-9)
 };
 
 // Source rows of a wave's copies of one token tile: the rows of its three
@@ -903,61 +553,95 @@ __device__ __forceinline__ void x8_rows(int (&rw)[4], const GArgs& g, int off, i
     rw[3] = src(32 * wave + (lane >> 1));
 }
 
-template <int MODE, class W>
-__device__ __forceinline__ void x8_plan_rows(XCopies& c, const GArgs& g, const W& w, int e, int n0, int mrows,
+template <int MODE, bool RG, class W>
+__device__ __forceinline__ void x8_plan_rows(XCopies<RG>& c, const GArgs& g, const W& w, int e, int n0, int mrows,
                                              const int (&rw)[4], int wave, int lane) {
     const uint32_t cbytes = (uint32_t)g.Kp >> 1, nch = (uint32_t)g.Kp >> 5;
     const int slot = lane & 7;
     c.na = (mrows + 63) >> 6;
     auto row_of = [&](int v) { return MODE == MODE_GATEUP ? v / g.topk : v; };
-    c.ars = mx::buf_rsrc(g.aq, (int64_t)g.a_rows * cbytes);
+    const uint32_t ald = RG ? (uint32_t)g.ald : cbytes, asld = RG ? (uint32_t)g.asld : nch;
+    c.ars = mx::buf_rsrc(g.aq, (int64_t)g.a_rows * ald);
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         const int r = 64 * j + 8 * wave + (lane >> 3);   // block 8j + wave
-        c.avo[j] = (uint32_t)row_of(rw[j]) * cbytes + ((slot ^ mx::swz_key128(r)) << 4);
+        c.avo[j] = (uint32_t)row_of(rw[j]) * ald + ((slot ^ mx::swz_key128(r)) << 4);
     }
-    // weight blocks 4*wave + j: rows 32*wave .. +31, one projection
+    // weight blocks 4*wave + j: rows 32*wave .. +31, one projection (RG: relative to row n0)
     int proj;
     weight_row<MODE>(32 * wave, n0, proj);
-    c.wrs = mx::buf_rsrc(w.p(e, proj), (int64_t)g.Nw * cbytes);
-    c.swrs = mx::buf_rsrc(w.s(e, proj), (int64_t)g.Nw * nch);
+    const int nbase = RG ? n0 : 0;
+    const int64_t wrows = RG ? min(g.Nw - n0, X_BN) : g.Nw;
+    c.wrs = mx::buf_rsrc(w.p(e, proj) + (int64_t)nbase * cbytes, wrows * cbytes);
+    auto rel_row = [&](int rho) {
+        int pj;
+        return (uint32_t)(min(weight_row<MODE>(rho, n0, pj), g.Nw - 1) - nbase);
+    };
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int rho = 32 * wave + 8 * j + (lane >> 3);
-        int pj;
-        const int rr = min(weight_row<MODE>(rho, n0, pj), g.Nw - 1);
-        c.wvo[j] = (uint32_t)rr * cbytes + ((slot ^ mx::swz_key128(rho)) << 4);
+        c.wvo[j] = rel_row(rho) * cbytes + ((slot ^ mx::swz_key128(rho)) << 4);
     }
-    {   // scale copies: lane -> row 32 * wave + lane / 2, 4 of its 8 bytes
-        const int row = 32 * wave + (lane >> 1);
-        int pj;
-        const int rr = min(weight_row<MODE>(row, n0, pj), g.Nw - 1);
-        c.swvo = (uint32_t)rr * nch + 4 * (lane & 1);
-        c.sars = mx::buf_rsrc(g.as, (int64_t)g.a_rows * nch);
-        c.savo = (uint32_t)row_of(rw[3]) * nch + 4 * (lane & 1);
+    // scale copies: lane -> row 32 * wave + lane / 2, 4 of its 8 bytes
+    c.sars = mx::buf_rsrc(g.as, (int64_t)g.a_rows * asld);
+    c.savo = (uint32_t)row_of(rw[3]) * asld + 4 * (lane & 1);
+    const uint8_t* sw = w.s(e, proj) + (int64_t)nbase * nch;
+    if constexpr (RG) {
+        const uint32_t d = (uint32_t)(uintptr_t)sw & 3u;
+        c.swrs = mx::buf_rsrc(sw - d, (wrows * nch + d + 3) & ~3ll);
+        c.swvo = ((rel_row(32 * wave + (lane >> 1)) * nch + d) & ~3u) + 4 * (lane & 1);
+        // the rows this lane's operand reads will take: 64 * (wave % 4) + 32 j + lane % 32
+        auto shift = [&](int j) {
+            const uint32_t rr = rel_row(64 * (wave & 3) + 32 * j + (lane & 31));
+            return (rr * nch + (uint32_t)(uintptr_t)w.s(e, MODE == MODE_GATEUP ? j : 2)) & 3u;
+        };
+        c.swvo2 = ((rel_row(32 * wave + (lane & 31)) * nch + d) & ~3u) + 8;
+        c.shw = shift(0) | (shift(1) << 8);
+    } else {
+        c.swrs = mx::buf_rsrc(sw, wrows * nch);
+        c.swvo = rel_row(32 * wave + (lane >> 1)) * nch + 4 * (lane & 1);
     }
 }
 
 // The token-row copies of K step s into the token stage at `abuf`, part
 // `part` (parts 0-1), and the weight-row copies of step s into the weight
 // stage at `wbuf`, part `part` (parts 2-3): within a step all token copies
-// come first and the last five are the weight copies.
-__device__ __forceinline__ void x8_issue_a(const XCopies& c, uint32_t abuf, int s, int part, int wave) {
+// come first and the last XL::WCP are the weight copies.  `left` (RG): the
+// row's 32-blocks from this step on.
+// Bit 31 set for a lane whose chunk of a row (r mod 16 of them) lies past the
+// row's end: an offset out of every range, the copy writes zeros.
+template <bool RG>
+__device__ __forceinline__ uint32_t past_end(int r, int left) {
+    if (!RG || left >= 8) return 0u;   // uniform
+    const int slot = threadIdx.x & 7;
+    return (slot ^ mx::swz_key128(r)) >= left ? 0x80000000u : 0u;
+}
+
+template <bool RG>
+__device__ __forceinline__ void x8_issue_a(const XCopies<RG>& c, uint32_t abuf, int s, int part, int wave, int left) {
     const uint32_t kofs = (uint32_t)s * X_ROWB;
+    const uint32_t past = past_end<RG>(8 * wave + ((threadIdx.x & 63) >> 3), left);
     if (part == 0) {
-        if (c.na > 0) mx::dma16(c.avo[0], c.ars, kofs, abuf + wave * 1024);
-        if (c.na > 1) mx::dma16(c.avo[1], c.ars, kofs, abuf + (8 + wave) * 1024);
+        if (c.na > 0) mx::dma16(c.avo[0] | past, c.ars, kofs, abuf + wave * 1024);
+        if (c.na > 1) mx::dma16(c.avo[1] | past, c.ars, kofs, abuf + (8 + wave) * 1024);
         if (wave < 2 * c.na) mx::dma4(c.savo, c.sars, (uint32_t)s * 8, abuf + X_A + 256 * wave);
     } else if (c.na > 2) {
-        mx::dma16(c.avo[2], c.ars, kofs, abuf + (16 + wave) * 1024);
+        mx::dma16(c.avo[2] | past, c.ars, kofs, abuf + (16 + wave) * 1024);
     }
 }
-__device__ __forceinline__ void x8_issue_w(const XCopies& c, uint32_t wbuf, int s, int part, int wave) {
+template <bool RG>
+__device__ __forceinline__ void x8_issue_w(const XCopies<RG>& c, uint32_t wbuf, int s, int part, int wave, int left) {
     const uint32_t kofs = (uint32_t)s * X_ROWB;
     const int j0 = 2 * (part - 2);
-    mx::dma16(c.wvo[j0], c.wrs, kofs, wbuf + (4 * wave + j0) * 1024);
-    mx::dma16(c.wvo[j0 + 1], c.wrs, kofs, wbuf + (4 * wave + j0 + 1) * 1024);
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+        mx::dma16(c.wvo[j0 + p] | past_end<RG>(8 * p + ((threadIdx.x & 63) >> 3), left), c.wrs, kofs,
+                  wbuf + (4 * wave + j0 + p) * 1024);
     if (part == 2) mx::dma4(c.swvo, c.swrs, (uint32_t)s * 8, wbuf + X_W + 256 * wave);
+    if constexpr (RG) {
+        if (part == 3 && (threadIdx.x & 63) < 32)
+            mx::dma4(c.swvo2, c.swrs, (uint32_t)s * 8, wbuf + X_W + 8 * X_BN + 128 * wave);
+    }
 }
 
 // ------------------------------------------------------------------ persistent 192 x 256 tiles
@@ -991,25 +675,15 @@ __device__ __forceinline__ void x8_issue_w(const XCopies& c, uint32_t wbuf, int 
 //    all of them.  The loads of a tile (the next tile's source rows, the
 //    queue atomic, the down tile's pair indices and weights) are issued at
 //    its start and used only after its K loop, where no copy is in flight.
-constexpr int XP_TROW = 136;                                // down transpose: 128 B + 8 per row
-static_assert(8 * 32 * XP_TROW <= X_WST, "the down transposes fit weight stage 0");
-constexpr int XP_MAXJ = kMaxExperts / 8;                    // experts per group
-constexpr int XP_UCUM = X_LDS;                              // int[XP_MAXJ + 1]: units of the experts below j
-constexpr int XP_ECNT = XP_UCUM + 4 * (XP_MAXJ + 1);        // int[XP_MAXJ]: expert counts
-constexpr int XP_EOFF = XP_ECNT + 4 * XP_MAXJ;              // int[XP_MAXJ]: expert offsets
-constexpr int XP_SLOT = XP_EOFF + 4 * XP_MAXJ;              // int: the unit the queue handed out
-constexpr int XP_LDS = XP_SLOT + 16;
-static_assert(XP_LDS <= 160 * 1024 && XP_MAXJ <= 128, "xp LDS layout (two experts per lane in the prefix)");
-
 struct XpTile {
     int e, n0, off, mt, mrows;
 };
 
 // The tile of unit u (uniform): the expert j of the group with
 // ucum[j] <= u < ucum[j+1], found by a ballot over the group's experts.
-template <int MODE>
+template <int MODE, bool RG>
 __device__ __forceinline__ XpTile xp_tile_of(const uint8_t* smem, int grp, int nj, int ntiles, int u, int lane) {
-    const int* ucum = reinterpret_cast<const int*>(smem + XP_UCUM);
+    const int* ucum = reinterpret_cast<const int*>(smem + XL<RG>::UCUM);
     int j = 0;
     for (int b = 0; b < nj; b += 64) {
         const int jj = b + lane;
@@ -1026,8 +700,8 @@ __device__ __forceinline__ XpTile xp_tile_of(const uint8_t* smem, int grp, int n
     const int nt = local - mti * ntiles;
     XpTile t;
     t.e = grp + 8 * j;
-    t.off = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(smem + XP_EOFF)[j]);
-    const int cnt = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(smem + XP_ECNT)[j]);
+    t.off = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(smem + XL<RG>::EOFF)[j]);
+    const int cnt = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(smem + XL<RG>::ECNT)[j]);
     t.mt = __builtin_amdgcn_readfirstlane(mti * X_BM);
     t.mrows = min(X_BM, cnt - t.mt);
     t.n0 = __builtin_amdgcn_readfirstlane(nt * (MODE == MODE_GATEUP ? X_BN / 2 : X_BN));
@@ -1041,27 +715,26 @@ __device__ __forceinline__ XpTile xp_tile_of(const uint8_t* smem, int grp, int n
 // waits for the plan's loads) are complete before the first copy is
 // issued: a wait placed after a copy would also wait for the copy, which
 // the compiler does not count.
-__device__ __forceinline__ void xp_prologue_part(XCopies& c, uint32_t ring, int nsteps, int wave, int part) {
+template <bool RG>
+__device__ __forceinline__ void xp_prologue_part(XCopies<RG>& c, uint32_t ring, int nch, int wave, int part) {
+    using L = XL<RG>;
     if (part == 0) {
         asm volatile("" : "+v"(c.avo[0]), "+v"(c.avo[1]), "+v"(c.avo[2]), "+v"(c.savo), "+v"(c.wvo[0]),
                      "+v"(c.wvo[1]), "+v"(c.wvo[2]), "+v"(c.wvo[3]), "+v"(c.swvo), "+s"(c.ars), "+s"(c.wrs),
                      "+s"(c.sars), "+s"(c.swrs) :: "memory");
-        x8_issue_w(c, ring + X_WST, 0, 2, wave);
-        x8_issue_w(c, ring + X_WST, 0, 3, wave);
+        if constexpr (RG) asm volatile("" : "+v"(c.swvo2), "+v"(c.shw) :: "memory");
+        x8_issue_w<RG>(c, ring + L::WST, 0, 2, wave, nch);
+        x8_issue_w<RG>(c, ring + L::WST, 0, 3, wave, nch);
     } else if (part == 1) {
-        x8_issue_a(c, ring + X_ARING, 0, 0, wave);
-        x8_issue_a(c, ring + X_ARING, 0, 1, wave);
-    } else if (nsteps > 1) {
-        x8_issue_w(c, ring + 2 * X_WST, 1, 2, wave);
-        x8_issue_w(c, ring + 2 * X_WST, 1, 3, wave);
+        x8_issue_a<RG>(c, ring + L::ARING, 0, 0, wave, nch);
+        x8_issue_a<RG>(c, ring + L::ARING, 0, 1, wave, nch);
+    } else if (nch > 8) {
+        x8_issue_w<RG>(c, ring + 2 * L::WST, 1, 2, wave, nch - 8);
+        x8_issue_w<RG>(c, ring + 2 * L::WST, 1, 3, wave, nch - 8);
     }
 }
 
-__device__ __forceinline__ void xp_prologue(XCopies& c, uint32_t ring, int nsteps, int wave) {
-    for (int part = 0; part < 3; ++part) xp_prologue_part(c, ring, nsteps, wave, part);
-}
-
-template <int MODE, int NB, class Issue>
+template <int MODE, bool RG, int NB, class Issue>
 __device__ __forceinline__ void xp_epilogue(mx::v16f (&acc)[3][2], const GArgs& g, uint8_t* smem, const XpTile& t,
                                             int wave, int lane, Issue&& issue);
 
@@ -1073,13 +746,15 @@ __device__ __forceinline__ void xp_epilogue(mx::v16f (&acc)[3][2], const GArgs& 
 // for the memory pipeline to accept them.  (All copies after the epilogue
 // measured slower: their latency is then exposed.)
 // NB = the wave's 32-token blocks holding routed tokens (0..3).
-template <int MODE, int NB, class Sync, class Issue>
-__device__ __forceinline__ void xp_tile(const XCopies& c, const GArgs& g, uint8_t* smem, uint32_t ring,
+template <int MODE, bool RG, int NB, class Sync, class Issue>
+__device__ __forceinline__ void xp_tile(const XCopies<RG>& c, const GArgs& g, uint8_t* smem, uint32_t ring,
                                         const XpTile& t, int wave, int lane, Sync&& sync, Issue&& issue) {
     const int wm = wave >> 2, wn = wave & 3;
     const int lr = lane & 31, h = lane >> 5;
     const int key = mx::swz_key128(lr);
-    const int nsteps = g.Kp / 256;
+    using L = XL<RG>;
+    const int nch = g.Kp >> 5;
+    const int nsteps = (nch + 7) >> 3;
     mx::v16f acc[3][2];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -1092,24 +767,38 @@ __device__ __forceinline__ void xp_tile(const XCopies& c, const GArgs& g, uint8_
         // this wave's copies of step it have landed (the weights of step
         // it+1, issued last, may still be in flight) and its reads of step
         // it-1 are done; after the barrier every wave's
-        if (it + 1 < nsteps) asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
+        if (it + 1 < nsteps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(L::WCP) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         const bool more_a = it + 1 < nsteps, more_w = it + 2 < nsteps;
-        const uint8_t* wst = smem + ((it + 1) % 3) * X_WST;
-        const uint8_t* ast = smem + X_ARING + (it & 1) * X_AST;
-        const uint32_t anxt = ring + X_ARING + ((it + 1) & 1) * X_AST;
-        const uint32_t wnxt = ring + (it % 3) * X_WST;   // step it+2: stage (it+3) % 3, step it-1's
+        const uint8_t* wst = smem + ((it + 1) % 3) * L::WST;
+        const uint8_t* ast = smem + L::ARING + (it & 1) * X_AST;
+        const uint32_t anxt = ring + L::ARING + ((it + 1) & 1) * X_AST;
+        const uint32_t wnxt = ring + (it % 3) * L::WST;   // step it+2: stage (it+3) % 3, step it-1's
         const uint8_t* la = ast + (32 * wm + lr) * X_ROWB;
         const uint8_t* lw = wst + (wn * 64 + lr) * X_ROWB;
         const uint8_t* lsa = ast + X_A + (32 * wm + lr) * 8;
         const uint8_t* lsw = wst + X_W + (wn * 64 + lr) * 8;
         uint32_t sa[3], sb[2];
+        const int left = nch - 8 * it;   // 32-blocks of the row from this step on
+        uint32_t keep = 0xFFFFFFFFu;     // RG: the blocks 2 ks + h < left
+        if (RG && left < 8) keep = left + 1 - h >= 8 ? 0xFFFFFFFFu : (1u << (4 * ((left + 1 - h) & ~1))) - 1u;
 #pragma unroll
-        for (int i = 0; i < NB; ++i) sa[i] = scale_word(lsa + i * 64 * 8, h);
+        for (int i = 0; i < NB; ++i) {
+            const uint2 v = *reinterpret_cast<const uint2*>(lsa + i * 64 * 8);
+            sa[i] = scale_word<RG>(v.x, v.y, h, keep);
+        }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) sb[j] = scale_word(lsw + j * 32 * 8, h);
+        for (int j = 0; j < 2; ++j) {
+            uint2 v = *reinterpret_cast<const uint2*>(lsw + j * 32 * 8);
+            if constexpr (RG) {
+                const uint32_t v2 = *reinterpret_cast<const uint32_t*>(wst + X_W + 8 * X_BN + (wn * 64 + j * 32 + lr) * 4);
+                const uint32_t sh = j ? c.shw >> 8 : c.shw;   // alignbyte takes bits 0-1
+                v = make_uint2(__builtin_amdgcn_alignbyte(v.y, v.x, sh), __builtin_amdgcn_alignbyte(v2, v.y, sh));
+            }
+            sb[j] = scale_word<RG>(v.x, v.y, h, keep);
+        }
         uint4 af[2][3], bf[2][2];
         auto load = [&](int ks, int r) {
             const int koff = ((2 * ks + h) ^ key) << 4;
@@ -1123,9 +812,9 @@ __device__ __forceinline__ void xp_tile(const XCopies& c, const GArgs& g, uint8_
         for (int ks = 0; ks < 4; ++ks) {
             __builtin_amdgcn_sched_barrier(0);
             if (ks < 2) {
-                if (more_a) x8_issue_a(c, anxt, it + 1, ks, wave);
+                if (more_a) x8_issue_a<RG>(c, anxt, it + 1, ks, wave, left - 8);
             } else if (more_w) {
-                x8_issue_w(c, wnxt, it + 2, ks, wave);
+                x8_issue_w<RG>(c, wnxt, it + 2, ks, wave, left - 16);
             }
             if (NB > 0) {
                 if (ks + 1 < 4) load(ks + 1, (ks + 1) & 1);
@@ -1148,12 +837,12 @@ __device__ __forceinline__ void xp_tile(const XCopies& c, const GArgs& g, uint8_
         for (int j = 0; j < 2; ++j) mx::pin(acc[i][j]);
     sync();
     issue(0);
-    xp_epilogue<MODE, NB>(acc, g, smem, t, wave, lane, issue);
+    xp_epilogue<MODE, RG, NB>(acc, g, smem, t, wave, lane, issue);
 }
 
 // Epilogue of one wave's token blocks (NB of them) of tile t; issues parts 1
 // and 2 of the next tile's first copies between its blocks.
-template <int MODE, int NB, class Issue>
+template <int MODE, bool RG, int NB, class Issue>
 __device__ __forceinline__ void xp_epilogue(mx::v16f (&acc)[3][2], const GArgs& g, uint8_t* smem, const XpTile& t,
                                             int wave, int lane, Issue&& issue) {
     const int wm = wave >> 2, wn = wave & 3;
@@ -1169,8 +858,8 @@ __device__ __forceinline__ void xp_epilogue(mx::v16f (&acc)[3][2], const GArgs& 
         // writes 8 whole 128-byte row segments; rows 136 bytes apart make
         // the 8-byte writes of 32 lanes (one row each) hit distinct banks
         uint8_t* tb = smem + wave * 32 * XP_TROW;
-        const int* lp = reinterpret_cast<const int*>(smem + X_PP);
-        const float* ls = reinterpret_cast<const float*>(smem + X_PP + 4 * X_BM);
+        const int* lp = reinterpret_cast<const int*>(smem + XL<RG>::PP);
+        const float* ls = reinterpret_cast<const float*>(smem + XL<RG>::PP + 4 * X_BM);
         // lane: buffer row 8*st + lane/8 (tile row 64*i + 32*wm + 8*st +
         // lane/8), 16 bytes at column chunk lane%8
         const int ch = lane & 7;
@@ -1208,22 +897,20 @@ __device__ __forceinline__ void xp_epilogue(mx::v16f (&acc)[3][2], const GArgs& 
         if (NB == 1) issue(2);
         return;
     }
-    const int pp[2] = {0, 0};
-    const float ss[2] = {0.0f, 0.0f};
     if (NB >= 2) {
         mx::v16f sub[2][2] = {{acc[0][0], acc[0][1]}, {acc[1][0], acc[1][1]}};
-        tile_epilogue<MODE, 2>(sub, g, t.n0, t.off, t.mt, t.mrows, 32 * wm, wn, lr, h, pp, ss, 64);
+        gateup_epilogue<2>(sub, g, t.n0, t.off, t.mt, t.mrows, 32 * wm, wn, lr, h);
         issue(1);
     }
     if (NB == 1 || NB == 3) {
         mx::v16f sub[2][2] = {{acc[NB - 1][0], acc[NB - 1][1]}, {acc[NB - 1][0], acc[NB - 1][1]}};
-        tile_epilogue<MODE, 1>(sub, g, t.n0, t.off, t.mt, t.mrows, 64 * (NB - 1) + 32 * wm, wn, lr, h, pp, ss, 64);
+        gateup_epilogue<1>(sub, g, t.n0, t.off, t.mt, t.mrows, 64 * (NB - 1) + 32 * wm, wn, lr, h);
         if (NB == 1) issue(1);
     }
     issue(2);
 }
 
-template <int MODE, class W>
+template <int MODE, bool RG, class W>
 __global__ __launch_bounds__(X_THREADS, 1) void grouped_gemm_xp_kernel(GArgs g, W w, int ntiles, int n_exp,
                                                                        int* __restrict__ qctr) {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -1234,10 +921,10 @@ __global__ __launch_bounds__(X_THREADS, 1) void grouped_gemm_xp_kernel(GArgs g, 
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t ring = __builtin_amdgcn_readfirstlane(mx::lds_addr(smem));
-    int* ucum = reinterpret_cast<int*>(smem + XP_UCUM);
-    int* ecnt = reinterpret_cast<int*>(smem + XP_ECNT);
-    int* eoff = reinterpret_cast<int*>(smem + XP_EOFF);
-    int* slot = reinterpret_cast<int*>(smem + XP_SLOT);
+    int* ucum = reinterpret_cast<int*>(smem + XL<RG>::UCUM);
+    int* ecnt = reinterpret_cast<int*>(smem + XL<RG>::ECNT);
+    int* eoff = reinterpret_cast<int*>(smem + XL<RG>::EOFF);
+    int* slot = reinterpret_cast<int*>(smem + XL<RG>::SLOT);
     const int nj = n_exp > grp ? (n_exp - grp + 7) / 8 : 0;
     if (nj == 0) return;
     for (int j = tid; j < nj; j += X_THREADS) {
@@ -1265,15 +952,15 @@ __global__ __launch_bounds__(X_THREADS, 1) void grouped_gemm_xp_kernel(GArgs g, 
     // units kw and kw + per are this workgroup's first two; the queue hands
     // out the rest, from 2 * per on
     if (kw >= nunits) return;
-    const int nsteps = g.Kp / 256;
-    XpTile t = xp_tile_of<MODE>(smem, grp, nj, ntiles, kw, lane);
-    XCopies c;
+    const int nch = g.Kp >> 5;
+    XpTile t = xp_tile_of<MODE, RG>(smem, grp, nj, ntiles, kw, lane);
+    XCopies<RG> c;
     {
         int rw[4];
         x8_rows<MODE>(rw, g, t.off, t.mt, t.mrows, wave, lane);
-        x8_plan_rows<MODE>(c, g, w, t.e, t.n0, t.mrows, rw, wave, lane);
+        x8_plan_rows<MODE, RG>(c, g, w, t.e, t.n0, t.mrows, rw, wave, lane);
     }
-    xp_prologue(c, ring, nsteps, wave);
+    for (int part = 0; part < 3; ++part) xp_prologue_part<RG>(c, ring, nch, wave, part);
     int un1 = kw + per;                          // the next tile's unit (uniform)
     const int trow = wave * 64 + lane;
     for (;;) {
@@ -1289,7 +976,7 @@ __global__ __launch_bounds__(X_THREADS, 1) void grouped_gemm_xp_kernel(GArgs g, 
         XpTile tn = t;
         int rwn[4];
         if (more) {
-            tn = xp_tile_of<MODE>(smem, grp, nj, ntiles, un1, lane);
+            tn = xp_tile_of<MODE, RG>(smem, grp, nj, ntiles, un1, lane);
             x8_rows<MODE>(rwn, g, tn.off, tn.mt, tn.mrows, wave, lane);
         }
         int uq;
@@ -1301,11 +988,11 @@ __global__ __launch_bounds__(X_THREADS, 1) void grouped_gemm_xp_kernel(GArgs g, 
             rp = g.pairs[r];
             rs = g.sscore[r];
         }
-        XCopies cn = c;
+        XCopies<RG> cn = c;
         auto sync = [&]() {
             if (MODE == MODE_DOWN && trow < t.mrows) {
-                reinterpret_cast<int*>(smem + X_PP)[trow] = rp;
-                reinterpret_cast<float*>(smem + X_PP + 4 * X_BM)[trow] = rs;
+                reinterpret_cast<int*>(smem + XL<RG>::PP)[trow] = rp;
+                reinterpret_cast<float*>(smem + XL<RG>::PP + 4 * X_BM)[trow] = rs;
             }
             if (tid == 0) *slot = uq;
             // every wave is past its last operand read of this tile (the
@@ -1317,17 +1004,17 @@ __global__ __launch_bounds__(X_THREADS, 1) void grouped_gemm_xp_kernel(GArgs g, 
         };
         auto issue = [&](int part) {
             if (more) {
-                if (part == 0) x8_plan_rows<MODE>(cn, g, w, tn.e, tn.n0, tn.mrows, rwn, wave, lane);
-                xp_prologue_part(cn, ring, nsteps, wave, part);
+                if (part == 0) x8_plan_rows<MODE, RG>(cn, g, w, tn.e, tn.n0, tn.mrows, rwn, wave, lane);
+                xp_prologue_part<RG>(cn, ring, nch, wave, part);
             }
         };
         // the wave's token blocks 2i + wm (i < nb) holding routed rows
         const int nb = min(((t.mrows + 31) / 32 - (wave >> 2) + 1) >> 1, 3);
         switch (nb) {
-            case 3: xp_tile<MODE, 3>(c, g, smem, ring, t, wave, lane, sync, issue); break;
-            case 2: xp_tile<MODE, 2>(c, g, smem, ring, t, wave, lane, sync, issue); break;
-            case 1: xp_tile<MODE, 1>(c, g, smem, ring, t, wave, lane, sync, issue); break;
-            default: xp_tile<MODE, 0>(c, g, smem, ring, t, wave, lane, sync, issue); break;
+            case 3: xp_tile<MODE, RG, 3>(c, g, smem, ring, t, wave, lane, sync, issue); break;
+            case 2: xp_tile<MODE, RG, 2>(c, g, smem, ring, t, wave, lane, sync, issue); break;
+            case 1: xp_tile<MODE, RG, 1>(c, g, smem, ring, t, wave, lane, sync, issue); break;
+            default: xp_tile<MODE, RG, 0>(c, g, smem, ring, t, wave, lane, sync, issue); break;
         }
         if (!more) break;
         un1 = 2 * per + __builtin_amdgcn_readfirstlane(*slot);
@@ -1372,6 +1059,7 @@ struct WsLayout {
 };
 
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+inline int64_t pad256(int v) { return ((int64_t)v + 255) & ~(int64_t)255; }
 
 // CUs per XCD of the current device (its CU count / 8), cached per device:
 // the persistent grouped GEMMs launch one workgroup per CU.
@@ -1389,6 +1077,7 @@ int cus_per_xcd() {
 
 WsLayout ws_layout(int T, int topk, int n_exp, int H, int Mi) {
     const size_t P = (size_t)T * topk;
+    const size_t Hp = pad256(H), Mp = pad256(Mi);   // the launch's own rows: whole K steps
     WsLayout L;
     size_t o = 0;
     L.counts = o; o = align256(o + sizeof(int) * n_exp);
@@ -1397,44 +1086,49 @@ WsLayout ws_layout(int T, int topk, int n_exp, int H, int Mi) {
     L.sscore = o; o = align256(o + sizeof(float) * P);
     L.hist = o;   o = align256(o + sizeof(int) * ((P + kRtChunk - 1) / kRtChunk) * n_exp);
     L.qctr = o;   o = align256(o + sizeof(int) * 16);
-    L.xq = o;     o = align256(o + (size_t)T * (H / 2));
-    L.xs = o;     o = align256(o + (size_t)T * (H / 32));
-    L.hq = o;     o = align256(o + P * (Mi / 2));
-    L.hs = o;     o = align256(o + P * (Mi / 32));
+    L.xq = o;     o = align256(o + (size_t)T * (Hp / 2));
+    L.xs = o;     o = align256(o + (size_t)T * (Hp / 32));
+    L.hq = o;     o = align256(o + P * (Mp / 2));
+    L.hs = o;     o = align256(o + P * (Mp / 32));
     L.yd = o;     o = align256(o + P * H * sizeof(uint16_t));
     L.total = o;
     return L;
 }
 
-template <class W>
-int run_prefill(const void* x, const int64_t* topi, const uint16_t* scores, W w, int n_exp, int T, int topk,
-                int H, int Mi, void* out, void* workspace, size_t ws_bytes, hipStream_t st) {
-    MXH_REQUIRE(x && topi && scores && out && workspace, "moe_prefill: null pointer");
-    MXH_REQUIRE(T > 0 && topk > 0 && topk <= kMaxTopk, "moe_prefill: T=%d topk=%d (need T > 0, 0 < topk <= %d)",
-                T, topk, kMaxTopk);
-    MXH_REQUIRE(n_exp > 0 && n_exp <= kMaxExperts, "moe_prefill: n_experts=%d (1..%d)", n_exp, kMaxExperts);
-    MXH_REQUIRE(H > 0 && H % 32 == 0 && Mi > 0 && Mi % 32 == 0,
-                "moe_prefill: H=%d and Mi=%d must be positive multiples of 32", H, Mi);
-    MXH_REQUIRE((int64_t)T * topk < (1ll << 31) / 2, "moe_prefill: T*topk too large");
-    MXH_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)workspace & 255) == 0,
-                "moe_prefill: x/out must be 16-byte and workspace 256-byte aligned");
-    const WsLayout L = ws_layout(T, topk, n_exp, H, Mi);
-    MXH_REQUIRE(ws_bytes >= L.total, "moe_prefill: workspace of %zu bytes < required %zu", ws_bytes, L.total);
-    static bool attr_set[2][6] = {};
-    constexpr int tw = std::is_same<W, TableW>::value ? 1 : 0;
-    for (int m = 0; m < 6; ++m) {
-        if (attr_set[tw][m]) continue;
-        const void* fns[6] = {reinterpret_cast<const void*>(grouped_gemm_kernel<MODE_GATEUP, W>),
-                              reinterpret_cast<const void*>(grouped_gemm_kernel<MODE_DOWN, W>),
-                              reinterpret_cast<const void*>(grouped_gemm_dma_kernel<MODE_GATEUP, W>),
-                              reinterpret_cast<const void*>(grouped_gemm_dma_kernel<MODE_DOWN, W>),
-                              reinterpret_cast<const void*>(grouped_gemm_xp_kernel<MODE_GATEUP, W>),
-                              reinterpret_cast<const void*>(grouped_gemm_xp_kernel<MODE_DOWN, W>)};
-        const int bytes = m < 2 ? 2 * BUF_BYTES : m < 4 ? D_NST * D_STAGE : XP_LDS;
-        hipError_t e = hipFuncSetAttribute(fns[m], hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-        MXH_REQUIRE(e == hipSuccess, "moe_prefill: cannot reserve %d B of LDS: %s", bytes, hipGetErrorString(e));
-        attr_set[tw][m] = true;
+// One kernel's LDS reservation, once per kernel and process.
+template <int MODE, bool RG, class W>
+int reserve_xp() {
+    static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(grouped_gemm_xp_kernel<MODE, RG, W>),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, XL<RG>::BYTES);
+    MXH_REQUIRE(e == hipSuccess, "moe_prefill: cannot reserve %d B of LDS: %s", XL<RG>::BYTES, hipGetErrorString(e));
+    return MXFP4_OK;
+}
+
+// A grouped GEMM over every expert's rows, one persistent workgroup per CU.
+template <int MODE, class W>
+int launch_xp(const GArgs& g, const W& w, int n_exp, int* qctr, hipStream_t st) {
+    const int per_tile = MODE == MODE_GATEUP ? X_BN / 2 : X_BN;
+    const int ntiles = (g.Nw + per_tile - 1) / per_tile;
+    const dim3 grid(8 * cus_per_xcd());
+    int rc;
+    // (without RG the weights are addressed with 32-bit offsets from the expert's first row)
+    if (g.Kp % 256 == 0 && (int64_t)g.Nw * (g.Kp / 2) < (1ll << 32)) {
+        if ((rc = reserve_xp<MODE, false, W>()) != MXFP4_OK) return rc;
+        hipLaunchKernelGGL((grouped_gemm_xp_kernel<MODE, false, W>), grid, dim3(X_THREADS), XL<false>::BYTES, st, g, w, ntiles,
+                           n_exp, qctr);
+    } else {
+        if ((rc = reserve_xp<MODE, true, W>()) != MXFP4_OK) return rc;
+        hipLaunchKernelGGL((grouped_gemm_xp_kernel<MODE, true, W>), grid, dim3(X_THREADS), XL<true>::BYTES, st, g, w, ntiles,
+                           n_exp, qctr);
     }
+    return mxh::launch_status(MODE == MODE_GATEUP ? "moe_prefill gate/up" : "moe_prefill down");
+}
+
+template <class W>
+int run_prefill_pass(const void* x, const int64_t* topi, const uint16_t* scores, W w, int n_exp, int T, int topk,
+                     int H, int Mi, void* out, void* workspace, hipStream_t st) {
+    const WsLayout L = ws_layout(T, topk, n_exp, H, Mi);
+    const int Hp = (int)pad256(H), Mp = (int)pad256(Mi);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     int* counts = reinterpret_cast<int*>(ws + L.counts);
     int* offs = reinterpret_cast<int*>(ws + L.offs);
@@ -1448,10 +1142,10 @@ int run_prefill(const void* x, const int64_t* topi, const uint16_t* scores, W w,
     // x -> fp16 -> MXFP4 once per token (the reference quantizes each gathered
     // copy; the bytes are identical), in the same launch: quantize_rows_kernel's
     // layout (x is 16-byte aligned and H a multiple of 32, so the vector path)
-    XQuant xqa{x, T, H, 2, 0, ws + L.xq, ws + L.xs};
-    while ((1 << xqa.lt) < H / 8 && xqa.lt < 8) ++xqa.lt;
+    XQuant xqa{x, T, H, Hp, 2, 0, ws + L.xq, ws + L.xs};
+    while ((1 << xqa.lt) < Hp / 8 && xqa.lt < 8) ++xqa.lt;
     xqa.gx = (T + (256 >> xqa.lt) - 1) / (256 >> xqa.lt);
-    const int xq_gy = (H / 8 + (1 << xqa.lt) - 1) >> xqa.lt;
+    const int xq_gy = (Hp / 8 + (1 << xqa.lt) - 1) >> xqa.lt;
     hipLaunchKernelGGL(route_count_kernel, dim3(nchunk + xqa.gx * xq_gy), dim3(64 * kRtWaves), 0, st, topi, P, n_exp,
                        hist, qctr, nchunk, xqa);
     hipLaunchKernelGGL(route_scatter_kernel, dim3(nchunk), dim3(64 * kRtWaves), 0, st, topi, P, n_exp, hist, counts,
@@ -1466,47 +1160,29 @@ int run_prefill(const void* x, const int64_t* topi, const uint16_t* scores, W w,
     g.topk = topk;
     g.hq = ws + L.hq;
     g.hs = ws + L.hs;
+    g.hld = Mp / 2;
+    g.hsld = Mp / 32;
     g.yd = reinterpret_cast<uint16_t*>(ws + L.yd);
     g.sscore = sscore;
 
     g.aq = ws + L.xq;
     g.as = ws + L.xs;
+    g.ald = Hp / 2;
+    g.asld = Hp / 32;
     g.Kp = H;
     g.Nw = Mi;
     g.a_rows = T;
-    // the copy kernels address operands with 32-bit byte offsets
-    const bool fit_gu = (int64_t)T * (H / 2) < (1ll << 32) && (int64_t)Mi * (H / 2) < (1ll << 32);
-    const bool fit_dn = (int64_t)P * (Mi / 2) < (1ll << 32) && (int64_t)H * (Mi / 2) < (1ll << 32);
-    const int xp_grid = 8 * cus_per_xcd();   // one persistent workgroup per CU
-    if (H % 256 == 0 && fit_gu) {
-        const int ntiles = (Mi + X_BN / 2 - 1) / (X_BN / 2);
-        hipLaunchKernelGGL((grouped_gemm_xp_kernel<MODE_GATEUP, W>), dim3(xp_grid), dim3(X_THREADS), XP_LDS, st, g,
-                           w, ntiles, n_exp, qctr);
-    } else if (H % DK == 0 && fit_gu)
-        hipLaunchKernelGGL((grouped_gemm_dma_kernel<MODE_GATEUP, W>), dim3((Mi + 63) / 64, n_exp), dim3(256),
-                           D_NST * D_STAGE, st, g, w);
-    else
-        hipLaunchKernelGGL((grouped_gemm_kernel<MODE_GATEUP, W>), dim3((Mi + 63) / 64, n_exp), dim3(256),
-                           2 * BUF_BYTES, st, g, w);
-    rc = mxh::launch_status("moe_prefill gate/up");
+    rc = launch_xp<MODE_GATEUP>(g, w, n_exp, qctr, st);
     if (rc != MXFP4_OK) return rc;
 
     g.aq = ws + L.hq;
     g.as = ws + L.hs;
+    g.ald = Mp / 2;
+    g.asld = Mp / 32;
     g.Kp = Mi;
     g.Nw = H;
     g.a_rows = P;
-    if (Mi % 256 == 0 && fit_dn) {
-        const int ntiles = (H + X_BN - 1) / X_BN;
-        hipLaunchKernelGGL((grouped_gemm_xp_kernel<MODE_DOWN, W>), dim3(xp_grid), dim3(X_THREADS), XP_LDS, st, g,
-                           w, ntiles, n_exp, qctr + 8);
-    } else if (Mi % DK == 0 && fit_dn)
-        hipLaunchKernelGGL((grouped_gemm_dma_kernel<MODE_DOWN, W>), dim3((H + BN - 1) / BN, n_exp), dim3(256),
-                           D_NST * D_STAGE, st, g, w);
-    else
-        hipLaunchKernelGGL((grouped_gemm_kernel<MODE_DOWN, W>), dim3((H + BN - 1) / BN, n_exp), dim3(256),
-                           2 * BUF_BYTES, st, g, w);
-    rc = mxh::launch_status("moe_prefill down");
+    rc = launch_xp<MODE_DOWN>(g, w, n_exp, qctr + 8, st);
     if (rc != MXFP4_OK) return rc;
 
     const int64_t threads = (int64_t)T * (H / 8);
@@ -1514,6 +1190,34 @@ int run_prefill(const void* x, const int64_t* topi, const uint16_t* scores, W w,
                        reinterpret_cast<const uint16_t*>(ws + L.yd), topi, T, topk, H, n_exp,
                        static_cast<uint16_t*>(out));
     return mxh::launch_status("moe_prefill combine");
+}
+
+template <class W>
+int run_prefill(const void* x, const int64_t* topi, const uint16_t* scores, W w, int n_exp, int T, int topk,
+                int H, int Mi, void* out, void* workspace, size_t ws_bytes, hipStream_t st) {
+    MXH_REQUIRE(x && topi && scores && out && workspace, "moe_prefill: null pointer");
+    MXH_REQUIRE(T > 0 && topk > 0 && topk <= kMaxTopk, "moe_prefill: T=%d topk=%d (need T > 0, 0 < topk <= %d)",
+                T, topk, kMaxTopk);
+    MXH_REQUIRE(n_exp > 0 && n_exp <= kMaxExperts, "moe_prefill: n_experts=%d (1..%d)", n_exp, kMaxExperts);
+    MXH_REQUIRE(H > 0 && H % 32 == 0 && Mi > 0 && Mi % 32 == 0,
+                "moe_prefill: H=%d and Mi=%d must be positive multiples of 32", H, Mi);
+    MXH_REQUIRE((int64_t)T * topk < (1ll << 31) / 2, "moe_prefill: T*topk too large");
+    MXH_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)workspace & 255) == 0,
+                "moe_prefill: x/out must be 16-byte and workspace 256-byte aligned");
+    MXH_REQUIRE(ws_bytes >= ws_layout(T, topk, n_exp, H, Mi).total, "moe_prefill: workspace of %zu bytes < required %zu",
+                ws_bytes, ws_layout(T, topk, n_exp, H, Mi).total);
+    // the copies address the token and h rows with 31-bit byte offsets: more
+    // tokens than that go in several passes, one after the other
+    const int64_t row = std::max(pad256(H) / 2, topk * (pad256(Mi) / 2));
+    MXH_REQUIRE(row < (1ll << 31), "moe_prefill: H=%d, topk=%d x Mi=%d too large", H, topk, Mi);
+    const int per = (int)std::min<int64_t>(T, ((1ll << 31) - 1) / row);
+    for (int t0 = 0; t0 < T; t0 += per) {
+        const int rc = run_prefill_pass<W>(static_cast<const uint8_t*>(x) + (int64_t)t0 * H * 2, topi + (int64_t)t0 * topk,
+                                           scores + (int64_t)t0 * topk, w, n_exp, std::min(per, T - t0), topk, H, Mi,
+                                           static_cast<uint8_t*>(out) + (int64_t)t0 * H * 2, workspace, st);
+        if (rc != MXFP4_OK) return rc;
+    }
+    return MXFP4_OK;
 }
 
 }  // namespace

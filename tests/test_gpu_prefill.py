@@ -163,3 +163,31 @@ def test_moe_compute_config3b_full_shape(dext):
     torch.cuda.synchronize()
     log("  device done; oracle over 128 experts ...")
     check_prefill(out, x, ti, tv, oracle_experts(stack), "config 3b")
+
+
+# H and / or Mi not a multiple of 256: a tail of one block and of seven, scale rows that start at any byte, one K step
+# and several, experts with more than one token tile, several token blocks
+@pytest.mark.parametrize("T,k,n_exp,H,Mi,skew", [(700, 4, 8, 288, 992, True), (333, 3, 5, 2016, 32, False),
+                                                 (50, 8, 40, 1184, 416, False), (450, 2, 3, 736, 352, True)])
+def test_moe_compute_ragged_vs_oracle(dext, T, k, n_exp, H, Mi, skew):
+    test_moe_compute_vs_oracle(dext, T, k, n_exp, H, Mi, skew)
+
+
+def test_moe_compute_ragged_dict_form_any_scale_byte(dext):
+    """Ragged rows through the pointer table, with every scale tensor at
+    another byte of a dword, equal the stacked form bit for bit."""
+    n_exp, H, Mi, T, k = 6, 416, 224, 90, 3
+    stack = make_stack(dext, n_exp, H, Mi, seed=410)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(10)
+    x = torch.randn((T, H), generator=g, device=DEV).bfloat16()
+    ti, tv = route(g, T, n_exp, k)
+    d = {e: stack.expert(e) for e in range(n_exp)}
+    for e, spec in d.items():
+        for j, nm in enumerate(("gate", "up", "down")):
+            t = spec[nm]["wsc"]
+            by = (e + j) % 4
+            buf = torch.empty(t.numel() + 8, dtype=torch.uint8, device=DEV)[by:by + t.numel()].view(t.shape)
+            buf.copy_(t)
+            spec[nm]["wsc"] = buf
+    assert torch.equal(moe_layer.moe_compute(x, ti, tv, d), moe_layer.moe_compute(x, ti, tv, stack))
