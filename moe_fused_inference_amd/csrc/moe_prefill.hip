@@ -8,15 +8,15 @@
 //         y = forward(silu(g) * u, down_e).to(bf16)                 # fp32 h -> half -> MXFP4
 //         out.index_add_(0, idx, y * scores[idx, slots])
 // which issues 3 launches per active expert and syncs on torch.where, with
-// five stream-ordered launches and no host synchronisation:
+// four or five stream-ordered launches and no host synchronisation:
 //
-//   1. route_kernel       one workgroup per two experts: counts of the ids
-//                         equal to / below each expert, then a stable ballot
-//                         compaction of the (token, slot) pairs routed to it
-//                         in row-major order -- exactly torch.where's order.
-//   2. quantize_rows      h (T, H) bf16 -> fp16-rounded -> MXFP4, once per
+//   1. routing            a stable counting sort of the (token, slot) pairs by
+//                         expert, row-major within one -- exactly torch.where's
+//                         order: one launch, or two from kR1Max pairs on.
+//   2. quantization       h (T, H) bf16 -> fp16-rounded -> MXFP4, once per
 //                         token (the per-row quantization does not depend on
-//                         which expert gathers the row).
+//                         which expert gathers the row), as further workgroups
+//                         of the (first) routing launch.
 //   3. grouped GEMM, gate/up   tiles of (expert, up to 192 of its tokens, 128
 //                         features): A = gathered token rows, W = the gate
 //                         rows of the features + their up rows; the
@@ -41,11 +41,6 @@
 #include "mx_device.h"
 #include "mx_host.h"
 #include "quant_rows.h"
-
-namespace mxh {
-int quantize_rows_impl(const void* x, int src_dtype, int round_to_f16, int64_t ldx, int M, int K, int Kp,
-                       uint8_t* q, uint8_t* s, hipStream_t st);
-}
 
 namespace {
 
@@ -218,17 +213,21 @@ struct XQuant {
     uint8_t* s;         // (T, Kp/32)
 };
 
+// Quantizer workgroup `local` of 256 threads (tid < 256).
+__device__ __forceinline__ void xquant_block(const XQuant& xq, int local, int tid) {
+    const int bx = local % xq.gx, by = local / xq.gx;
+    const int64_t row = (int64_t)bx * (256 >> xq.lt) + (tid >> xq.lt);
+    const int u = by * (1 << xq.lt) + (tid & ((1 << xq.lt) - 1));
+    mxq::quantize_unit<MXFP4_DT_BF16, 1>(xq.x, xq.H, xq.T, xq.H, xq.Kp, true, row, u, xq.q, xq.s);
+}
+
 __global__ __launch_bounds__(64 * kRtWaves) void route_count_kernel(const int64_t* __restrict__ topi, int P, int n_exp,
                                                                    int* __restrict__ hist, int* __restrict__ qctr,
                                                                    int nchunk, XQuant xq) {
     __shared__ int h[kMaxExperts];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if ((int)blockIdx.x >= nchunk) {
-        const int local = (int)blockIdx.x - nchunk;
-        const int bx = local % xq.gx, by = local / xq.gx;
-        const int64_t row = (int64_t)bx * (256 >> xq.lt) + (tid >> xq.lt);
-        const int u = by * (1 << xq.lt) + (tid & ((1 << xq.lt) - 1));
-        mxq::quantize_unit<MXFP4_DT_BF16, 1>(xq.x, xq.H, xq.T, xq.H, xq.Kp, true, row, u, xq.q, xq.s);
+        xquant_block(xq, (int)blockIdx.x - nchunk, tid);
         return;
     }
     if (qctr && blockIdx.x == 0 && tid < 16) qctr[tid] = 0;   // the grouped GEMMs' tile queues (8 each)
@@ -352,6 +351,102 @@ __global__ __launch_bounds__(64 * kRtWaves) void route_scatter_kernel(const int6
         // after every lane has its position, the group leader moves the
         // wave's offset of this expert past the group
         if ((mk[k] & ((1ull << lane) - 1ull)) == 0) wh[wave][id[k]] += __popcll(mk[k]);
+    }
+}
+
+// Both launches in one for up to kR1Max pairs: workgroup 0 alone sorts, wave w
+// taking the w-th sixteenth of the pairs in 64-id groups; the workgroups past
+// it quantize x (four of the quantizer's blocks each).  What bounds it at these
+// sizes is latency, so a launch and the histograms' trip through memory saved
+// are worth a single workgroup's ballots (measured on MI355X, 100 tokens x 8:
+// count + scatter 4.3 + 5.4 us, 4.5 us here), which from kR1Max on are not (500
+// tokens: the call 92.0 and 90.1 us, the gain already down to 2 us).
+constexpr int kR1Waves = 16, kR1Groups = 4;
+constexpr int kR1Max = 64 * kR1Waves * kR1Groups;
+
+__global__ __launch_bounds__(64 * kR1Waves) void route_one_kernel(const int64_t* __restrict__ topi, int P, int n_exp,
+                                                                  int* __restrict__ qctr, int* __restrict__ counts,
+                                                                  int* __restrict__ offs, int* __restrict__ pairs,
+                                                                  const uint16_t* __restrict__ scores,
+                                                                  float* __restrict__ sscore, XQuant xq) {
+    __shared__ uint16_t wh[kR1Waves][kMaxExperts];   // per-wave counts, then exclusive prefix over waves
+    __shared__ int base[kMaxExperts];
+    __shared__ int wsum[kR1Waves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (blockIdx.x > 0) {
+        xquant_block(xq, 4 * ((int)blockIdx.x - 1) + (tid >> 8), tid & 255);
+        return;
+    }
+    if (tid < 16) qctr[tid] = 0;   // the grouped GEMMs' tile queues (8 each)
+    const int groups = (P + 64 * kR1Waves - 1) / (64 * kR1Waves);   // of 64 ids per wave, <= kR1Groups
+    const int p0 = wave * groups * 64 + lane;
+    int id[kR1Groups];
+    int64_t raw[kR1Groups];
+    uint16_t sc[kR1Groups];
+#pragma unroll
+    for (int k = 0; k < kR1Groups; ++k) {   // unconditional (clamped) loads: all in flight at once
+        const int p = min(p0 + 64 * k, P - 1);
+        raw[k] = topi[p];
+        sc[k] = scores[p];
+    }
+    for (int i = tid; i < kR1Waves * kMaxExperts / 2; i += 64 * kR1Waves) reinterpret_cast<uint32_t*>(wh)[i] = 0;
+    const int bits = id_bits(n_exp);
+    __syncthreads();
+    uint64_t mk[kR1Groups];
+    const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int k = 0; k < kR1Groups; ++k) {
+        id[k] = k < groups && p0 + 64 * k < P && raw[k] >= 0 && raw[k] < n_exp ? (int)raw[k] : -1;
+        mk[k] = 0;
+        if (k >= groups) continue;   // uniform
+        const bool valid = id[k] >= 0;
+        mk[k] = same_id_lanes(id[k], valid, bits);
+        if (valid && (mk[k] & below) == 0) wh[wave][id[k]] += (uint16_t)__popcll(mk[k]);   // one writer per expert and group
+    }
+    __syncthreads();
+    // thread e: expert e's prefix over the waves, then the scan over experts
+    int tot = 0;
+    if (tid < n_exp) {
+#pragma unroll
+        for (int w = 0; w < kR1Waves; ++w) {
+            const int v = wh[w][tid];
+            wh[w][tid] = (uint16_t)tot;
+            tot += v;
+        }
+    }
+    int incl = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(incl, o);
+        if (lane >= o) incl += t;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int run = 0;
+    for (int w = 0; w < wave; ++w) run += wsum[w];
+    if (tid < n_exp) {
+        base[tid] = run + incl - tot;
+        counts[tid] = tot;
+        offs[tid] = run + incl - tot;
+    }
+    __syncthreads();
+    for (int k = 0; k < groups; ++k) {
+        int e = -1, p = p0 + 64 * k;
+        uint64_t m = 0;
+        uint16_t s = 0;
+#pragma unroll
+        for (int q = 0; q < kR1Groups; ++q)
+            if (q == k) {
+                e = id[q];
+                m = mk[q];
+                s = sc[q];
+            }
+        if (e < 0) continue;
+        const int at = base[e] + wh[wave][e] + __popcll(m & below);
+        pairs[at] = p;
+        sscore[at] = mx::bf16_to_f32(s);
+        // after every lane has its position, the group leader moves the wave's offset past the group
+        if ((m & below) == 0) wh[wave][e] += (uint16_t)__popcll(m);
     }
 }
 
@@ -1023,7 +1118,15 @@ __global__ __launch_bounds__(X_THREADS, 1) void grouped_gemm_xp_kernel(GArgs g, 
     }
 }
 
-// out[t, c] = bf16(sum_{k < topk, id valid} yd[t*topk + k, c]); 8 columns per thread
+// out[t, c] = bf16(sum_{k < topk, id valid} yd[t*topk + k, c]); 8 columns per
+// thread.  K8 (topk <= 8): a token's ids and then its rows are all loaded
+// before any is used, two memory latencies instead of one per slot; from
+// kCombineFew workgroups on others cover them and the plain loop is as fast
+// (MI355X, 100 tokens x 8 of 2048: 6.4 us and 4.7; 2048 tokens 12.2 and
+// 12.6).
+constexpr int kCombineFew = 1024;
+
+template <bool K8>
 __global__ __launch_bounds__(256) void prefill_combine_kernel(const uint16_t* __restrict__ yd,
                                                               const int64_t* __restrict__ topi, int T, int topk,
                                                               int H, int n_exp, uint16_t* __restrict__ out) {
@@ -1035,15 +1138,31 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const uint16_t* __
     float s[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) s[i] = 0.0f;
-    for (int k = 0; k < topk; ++k) {
-        const int64_t id = topi[(int64_t)t * topk + k];
-        if (id < 0 || id >= n_exp) continue;
-        const uint4 v = *reinterpret_cast<const uint4*>(yd + ((int64_t)t * topk + k) * H + c);
+    auto add = [&](const uint4& v) {
         const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             s[2 * i] += mx::bf16_to_f32((uint16_t)(wv[i] & 0xFFFFu));
             s[2 * i + 1] += mx::bf16_to_f32((uint16_t)(wv[i] >> 16));
+        }
+    };
+    const uint16_t* row = yd + (int64_t)t * topk * H + c;
+    if constexpr (K8) {
+        int64_t id[8];
+        uint4 v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) id[k] = topi[(int64_t)t * topk + min(k, topk - 1)];
+        // (rows of invalid ids are loaded, never written, and left out)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const uint4*>(row + (int64_t)min(k, topk - 1) * H);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (k < topk && id[k] >= 0 && id[k] < n_exp) add(v[k]);
+    } else {
+        for (int k = 0; k < topk; ++k) {
+            const int64_t id = topi[(int64_t)t * topk + k];
+            if (id < 0 || id >= n_exp) continue;
+            add(*reinterpret_cast<const uint4*>(row + (int64_t)k * H));
         }
     }
     uint32_t o[4];
@@ -1146,10 +1265,15 @@ int run_prefill_pass(const void* x, const int64_t* topi, const uint16_t* scores,
     while ((1 << xqa.lt) < Hp / 8 && xqa.lt < 8) ++xqa.lt;
     xqa.gx = (T + (256 >> xqa.lt) - 1) / (256 >> xqa.lt);
     const int xq_gy = (Hp / 8 + (1 << xqa.lt) - 1) >> xqa.lt;
-    hipLaunchKernelGGL(route_count_kernel, dim3(nchunk + xqa.gx * xq_gy), dim3(64 * kRtWaves), 0, st, topi, P, n_exp,
-                       hist, qctr, nchunk, xqa);
-    hipLaunchKernelGGL(route_scatter_kernel, dim3(nchunk), dim3(64 * kRtWaves), 0, st, topi, P, n_exp, hist, counts,
-                       offs, pairs, scores, sscore);
+    if (P <= kR1Max) {
+        hipLaunchKernelGGL(route_one_kernel, dim3(1 + (xqa.gx * xq_gy + 3) / 4), dim3(64 * kR1Waves), 0, st, topi, P, n_exp,
+                           qctr, counts, offs, pairs, scores, sscore, xqa);
+    } else {
+        hipLaunchKernelGGL(route_count_kernel, dim3(nchunk + xqa.gx * xq_gy), dim3(64 * kRtWaves), 0, st, topi, P, n_exp,
+                           hist, qctr, nchunk, xqa);
+        hipLaunchKernelGGL(route_scatter_kernel, dim3(nchunk), dim3(64 * kRtWaves), 0, st, topi, P, n_exp, hist, counts,
+                           offs, pairs, scores, sscore);
+    }
     int rc = mxh::launch_status("moe_prefill route");
     if (rc != MXFP4_OK) return rc;
 
@@ -1186,9 +1310,10 @@ int run_prefill_pass(const void* x, const int64_t* topi, const uint16_t* scores,
     if (rc != MXFP4_OK) return rc;
 
     const int64_t threads = (int64_t)T * (H / 8);
-    hipLaunchKernelGGL(prefill_combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
-                       reinterpret_cast<const uint16_t*>(ws + L.yd), topi, T, topk, H, n_exp,
-                       static_cast<uint16_t*>(out));
+    const unsigned blocks = (unsigned)((threads + 255) / 256);
+    auto* combine = topk <= 8 && blocks < kCombineFew ? prefill_combine_kernel<true> : prefill_combine_kernel<false>;
+    hipLaunchKernelGGL(combine, dim3(blocks), dim3(256), 0, st, reinterpret_cast<const uint16_t*>(ws + L.yd), topi, T, topk, H,
+                       n_exp, static_cast<uint16_t*>(out));
     return mxh::launch_status("moe_prefill combine");
 }
 

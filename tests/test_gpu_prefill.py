@@ -191,3 +191,24 @@ def test_moe_compute_ragged_dict_form_any_scale_byte(dext):
             buf.copy_(t)
             spec[nm]["wsc"] = buf
     assert torch.equal(moe_layer.moe_compute(x, ti, tv, d), moe_layer.moe_compute(x, ti, tv, stack))
+
+
+# the one-launch routing: one pair, one 64-id group per wave and its neighbours, the most it takes and one token past
+# (two launches); more experts than ids, the largest number of experts; the eight-slot combine at fewer slots
+@pytest.mark.parametrize("T,k,n_exp", [(1, 1, 3), (128, 8, 8), (129, 8, 8), (512, 8, 16), (513, 8, 16), (17, 5, 1024), (60, 12, 40)])
+def test_moe_compute_routing_sizes(dext, T, k, n_exp):
+    """Some ids out of range: those slots contribute nothing (compared with
+    the same call on their valid slots' tokens by the oracle)."""
+    H, Mi = 256, 64
+    stack = make_stack(dext, n_exp, H, Mi, seed=900 + n_exp)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(T * 31 + k)
+    x = torch.randn((T, H), generator=g, device=DEV).bfloat16()
+    ti, tv = route(g, T, n_exp, k)
+    if T > 1:
+        ti[T // 2, 0] = -1
+        ti[T - 1, k - 1] = n_exp
+    out = moe_layer.moe_compute(x, ti, tv, stack)
+    torch.cuda.synchronize()
+    used = [e for e in range(n_exp) if bool((ti == e).any())]
+    check_prefill(out, x, ti, tv, oracle_experts(stack, used), f"routing T={T} k={k} n={n_exp}")
