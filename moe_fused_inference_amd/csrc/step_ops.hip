@@ -204,20 +204,33 @@ __global__ __launch_bounds__(256) void qk_rope_kv_kernel(const float* __restrict
 }
 
 // ------------------------------------------------------------------ greedy argmax
-// Workgroup (slice p of kArgSlice logits, row m): the first index of the
-// slice's maximum (NaNs never win) goes to the workspace; the workgroup that
-// finishes a row last (a counter per row) merges the row's slices, and the
-// one that finishes the last row advances dpos.  Every counter is put back
-// to zero by the workgroup that read it last, so the workspace needs one
-// zero fill when it is allocated and never again (graph replays included).
+// Workgroup (slice p of kArgSlice logits, row m): the slice's maximum and its
+// first index (NaNs never win) go into the row's 64-bit key by an atomic
+// maximum -- the logit's bits in an order of unsigned integers above, the
+// index's complement below, so the larger key is the larger logit or, of equal
+// ones, the smaller index; the workgroup that finishes a row last (a counter
+// per row) writes the row's index, and the one that finishes the last row
+// advances dpos.  Every key and counter is put back to zero by the workgroup
+// that read it last, so the workspace needs one zero fill when it is allocated
+// and never again (graph replays included).
+// Everything handed over goes through those atomics, each waited for before
+// the next, so no fence is needed: with the slices' results in memory, the
+// release and acquire of every workgroup wrote back and invalidated its XCD's
+// L2, 15.4 us for 8 x 151936 logits (MI355X) against 8.7 here.
 constexpr int kArgPer = 16;                  // logits per thread
 constexpr int kArgSlice = 256 * kArgPer;     // logits per workgroup
 
 struct ArgWs {
     uint32_t* cnt;   // (M) slices done per row, then 1 word: rows done
-    float* val;      // (M, P) slice maxima
-    int32_t* idx;    // (M, P) their indices
+    uint64_t* key;   // (M)
 };
+
+// The key of a logit that is not NaN (-0 as 0).
+__device__ __forceinline__ uint64_t arg_key(float v, int idx) {
+    const uint32_t b = __float_as_uint(v + 0.0f);
+    const uint32_t o = b ^ (b >> 31 ? 0xFFFFFFFFu : 0x80000000u);
+    return ((uint64_t)o << 32) | (uint32_t)~idx;
+}
 
 __device__ __forceinline__ void arg_better(float& best, int& idx, float ob, int oi) {
     if (ob > best || (ob == best && oi < idx)) {
@@ -236,7 +249,6 @@ __global__ __launch_bounds__(256) void argmax_kernel(const float* __restrict__ l
                                                      ArgWs ws) {
     __shared__ float bv[4];
     __shared__ int bi[4];
-    __shared__ int last;
     const int p = blockIdx.x, m = blockIdx.y, P = gridDim.x;
     const float* row = logits + (int64_t)m * V;
     const int base = p * kArgSlice;
@@ -277,34 +289,22 @@ __global__ __launch_bounds__(256) void argmax_kernel(const float* __restrict__ l
         bi[wave] = idx;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; ++w) arg_better(best, idx, bv[w], bi[w]);
-        ws.val[(int64_t)m * P + p] = best;
-        ws.idx[(int64_t)m * P + p] = idx;
-        __threadfence();
-        const uint32_t done = __hip_atomic_fetch_add(&ws.cnt[m], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        last = done == (uint32_t)(P - 1);
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < 4; ++w) arg_better(best, idx, bv[w], bi[w]);
+    if (idx != 0x7FFFFFFF) {   // a slice of NaNs and -inf has no say
+        const uint64_t old = __hip_atomic_fetch_max(&ws.key[m], arg_key(best, idx), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::"v"((uint32_t)old) : "memory");   // done before the count
     }
-    __syncthreads();
-    if (!last || wave != 0) return;
-    // the row's last workgroup: merge its P slices (wave 0)
-    const int lane = threadIdx.x & 63;
-    best = -INFINITY;
-    idx = 0x7FFFFFFF;
-    for (int q = lane; q < P; q += 64)
-        arg_better(best, idx, __hip_atomic_load(&ws.val[(int64_t)m * P + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                   __hip_atomic_load(&ws.idx[(int64_t)m * P + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    arg_wave(best, idx);
-    if (lane == 0) {
-        ids[m] = idx == 0x7FFFFFFF ? 0 : idx;
-        __hip_atomic_store(&ws.cnt[m], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (dpos) {
-            __threadfence();
-            const uint32_t rows = __hip_atomic_fetch_add(&ws.cnt[M], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-            if (rows == (uint32_t)(M - 1)) {
-                *dpos += M;
-                __hip_atomic_store(&ws.cnt[M], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+    const uint32_t done = __hip_atomic_fetch_add(&ws.cnt[m], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (done != (uint32_t)(P - 1)) return;
+    const uint64_t key = __hip_atomic_exchange(&ws.key[m], (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    ids[m] = key == 0 ? 0 : (int)~(uint32_t)key;
+    __hip_atomic_store(&ws.cnt[m], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (dpos) {
+        const uint32_t rows = __hip_atomic_fetch_add(&ws.cnt[M], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (rows == (uint32_t)(M - 1)) {
+            *dpos += M;
+            __hip_atomic_store(&ws.cnt[M], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
@@ -376,8 +376,7 @@ extern "C" int mxfp4_argmax_advance(const float* logits, int M, int V, int32_t* 
     const int P = (V + kArgSlice - 1) / kArgSlice;
     const int64_t head = ((int64_t)(M + 1) * 4 + 255) / 256 * 256;
     uint8_t* w = static_cast<uint8_t*>(ws);
-    ArgWs a{reinterpret_cast<uint32_t*>(w), reinterpret_cast<float*>(w + head),
-            reinterpret_cast<int32_t*>(w + head + (int64_t)M * P * 4)};
+    ArgWs a{reinterpret_cast<uint32_t*>(w), reinterpret_cast<uint64_t*>(w + head)};
     hipLaunchKernelGGL(argmax_kernel, dim3(P, M), dim3(256), 0, mxh::as_stream(stream), logits, V, M, ids, dpos, a);
     return mxh::launch_status("argmax_advance");
 }
