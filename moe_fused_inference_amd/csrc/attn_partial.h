@@ -13,12 +13,13 @@
 #include "kv_codec.h"
 #include "mx_device.h"
 
+#include <type_traits>
+
 namespace ap {
 
 using am::kChunk;
 using am::kD;
 using am::kPart;
-using kv::e4m3_ref_decode;
 
 constexpr int kMaxFusedM = 16;   // tokens per call of the fused entry (the decode step's M)
 
@@ -46,21 +47,15 @@ __device__ __forceinline__ mx::v4f mfma_bf16(uint4 a, uint4 b, mx::v4f c) {
                                                    0, 0, 0);
 }
 
-// A cache byte (the reference's codec) as bf16 bits: every value of the
-// codec, 840 included, is a bf16 value, so this is exact.
-__device__ __forceinline__ uint32_t kv_bf16(uint32_t b) { return __float_as_uint(e4m3_ref_decode(b)) >> 16; }
-__device__ __forceinline__ uint32_t pack_bf16(uint32_t lo, uint32_t hi) { return lo | (hi << 16); }
-// The same through a 256-entry LDS table of the codec's bf16 bits (lut[b]
-// = kv_bf16(b), built once per workgroup): one LDS read per byte instead of
-// the codec's ~12 instructions.
-__device__ __forceinline__ uint32_t kv_lut(const uint16_t* lut, uint32_t b) { return lut[b & 0xFFu]; }
-__device__ __forceinline__ uint4 kv8_bf16(const uint16_t* lut, uint2 w) {
-    return make_uint4(pack_bf16(kv_lut(lut, w.x), kv_lut(lut, w.x >> 8)),
-                      pack_bf16(kv_lut(lut, w.x >> 16), kv_lut(lut, w.x >> 24)),
-                      pack_bf16(kv_lut(lut, w.y), kv_lut(lut, w.y >> 8)),
-                      pack_bf16(kv_lut(lut, w.y >> 16), kv_lut(lut, w.y >> 24)));
+// Eight cache bytes (the reference's codec) of one row as bf16: every value of
+// the codec, 840 included, is a bf16 value, so this is exact.
+template <bool EXP15>
+__device__ __forceinline__ uint4 kv8_bf16(uint2 w, uint32_t& e15) {
+    uint32_t f0, f1;
+    const uint32_t a = kv::ready<EXP15>(w.x, f0, e15), b = kv::ready<EXP15>(w.y, f1, e15);
+    return make_uint4(kv::pair_of<false, false, EXP15>(a, f0), kv::pair_of<true, false, EXP15>(a, f0),
+                      kv::pair_of<false, false, EXP15>(b, f1), kv::pair_of<true, false, EXP15>(b, f1));
 }
-
 
 // The chunk pass's LDS.
 template <int RT, bool FUSED>
@@ -71,7 +66,6 @@ struct AttnLds {
     alignas(16) uint16_t plo[R][kChunk + 8];     // p - high, bf16
     float red[4][R];
     float rstat[2][R];
-    uint16_t lut[256];
     alignas(16) uint8_t knew[FUSED ? kChunk : 1][kD];
     alignas(16) uint8_t vnew[FUSED ? kChunk : 1][kD];
     float2 rcs[FUSED ? kMaxFusedM : 1][64];
@@ -103,8 +97,8 @@ struct PlainQkv {
 // query rows, row r = (token m0 + r / G, head g*G + r % G), all sharing the
 // chunk's K and V rows, which are loaded and decoded once.
 //  1. loads first: K bytes in the MFMA operand layout (wave w: positions
-//     16w..16w+15), V bytes likewise (wave w: columns 32w..32w+31, 8
-//     positions a lane), q rows to LDS; the position only masks (rows past
+//     16w..16w+15), V bytes likewise (wave w: columns 32w..32w+31, a lane two
+//     adjacent ones of 8 positions), q rows to LDS; the position only masks (rows past
 //     max_pos are clamped), so the workgroup pays one memory latency;
 //  2. S = Q K^T on MFMA (bf16 q, bf16-exact K, fp32 accumulation), the raw
 //     scores to sc;
@@ -149,8 +143,6 @@ __device__ __forceinline__ void attn_partial_body(AttnLds<RT, FUSED>& L, const Q
     auto& plo = L.plo;
     auto& red = L.red;
     auto& rstat = L.rstat;
-    auto& lut = L.lut;
-    lut[tid] = (uint16_t)kv_bf16((uint32_t)tid);   // 256 threads: one entry each
     // ---- 1. loads
     uint2 kraw[4];
     {
@@ -158,34 +150,57 @@ __device__ __forceinline__ void attn_partial_body(AttnLds<RT, FUSED>& L, const Q
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) kraw[kt] = *reinterpret_cast<const uint2*>(kr + kt * 32);
     }
-    uint32_t vraw[2][2][8];
+    uint32_t vraw[2][8];   // columns 32w + 2 l16, + 1 of eight positions
     {
-        const uint8_t* vc = kvv + g * kD + wave * 32 + l16;
+        const uint8_t* vc = kvv + g * kD + wave * 32 + 2 * l16;
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int t = 0; t < 8; ++t)
-                    vraw[c][kt][t] = vc[(int64_t)(s0 + min(kt * 32 + lq * 8 + t, rowmax)) * rs + c * 16];
+            for (int t = 0; t < 8; ++t)
+                vraw[kt][t] = *reinterpret_cast<const uint16_t*>(vc + (int64_t)(s0 + min(kt * 32 + lq * 8 + t, rowmax)) * rs);
     }
     const int base = *dpos;
-    // with a waiting q|k|v source: K / V as bf16 MFMA operands, decoded ahead
-    uint4 kdec[QSRC::kWaits ? 4 : 1], vdec[QSRC::kWaits ? 2 : 1][2];
-    auto decode_v = [&](int kt, int c) {
-        const uint32_t* v = vraw[c][kt];
-        return make_uint4(pack_bf16(kv_lut(lut, v[0]), kv_lut(lut, v[1])), pack_bf16(kv_lut(lut, v[2]), kv_lut(lut, v[3])),
-                          pack_bf16(kv_lut(lut, v[4]), kv_lut(lut, v[5])), pack_bf16(kv_lut(lut, v[6]), kv_lut(lut, v[7])));
-    };
-    auto decode_all = [&]() {
-        if constexpr (QSRC::kWaits) {
+    // tokens m0..m0+MT-1 sit at positions base + m; those inside [0, max_pos) count
+    const int mv_lo = max(m0, -base);
+    const int mv_hi = min(min(M, m0 + MT) - 1, max_pos - 1 - base);
+    // uniform: no token of this workgroup reaches the chunk (so none of their rows is in it either)
+    const bool idle = mv_hi < mv_lo || s0 > base + mv_hi;
+    if constexpr (!QSRC::kWaits)
+        if (idle) return;
+    // K / V as bf16 MFMA operands (with a waiting q|k|v source decoded ahead of
+    // the wait); bytes of exponent 15 send the wave through the longer decode
+    uint4 kdec[4], vdec[2][2];
+    auto decode_k = [&]() {
+        uint32_t e15 = 0;
 #pragma unroll
-            for (int kt = 0; kt < 4; ++kt) kdec[kt] = kv8_bf16(lut, kraw[kt]);
+        for (int kt = 0; kt < 4; ++kt) kdec[kt] = kv8_bf16<false>(kraw[kt], e15);
+        if (__ballot((e15 & 0x80808080u) != 0u)) {
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int c = 0; c < 2; ++c) vdec[kt][c] = decode_v(kt, c);
+            for (int kt = 0; kt < 4; ++kt) kdec[kt] = kv8_bf16<true>(kraw[kt], e15);
         }
+    };
+    // column c of the lane's pair, positions kt * 32 + lq * 8 + t: bytes (t, t + 1)
+    // of either column from one word
+    auto decode_v_as = [&](auto exp15, uint32_t& e15) {
+        constexpr bool E = decltype(exp15)::value;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+            uint32_t o[2][4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                uint32_t f;
+                const uint32_t w = kv::ready<E>(__builtin_amdgcn_perm(vraw[kt][2 * t + 1], vraw[kt][2 * t], 0x05010400u), f, e15);
+                o[0][t] = kv::pair_of<false, false, E>(w, f);
+                o[1][t] = kv::pair_of<true, false, E>(w, f);
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) vdec[kt][c] = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
+        }
+    };
+    auto decode_v = [&]() {
+        uint32_t e15 = 0;
+        decode_v_as(std::false_type{}, e15);
+        if (__ballot((e15 & 0x80808080u) != 0u)) decode_v_as(std::true_type{}, e15);
     };
     if (!FUSED) {
         for (int i = tid; i < R * 16; i += 256) {
@@ -238,8 +253,8 @@ __device__ __forceinline__ void attn_partial_body(AttnLds<RT, FUSED>& L, const Q
         if constexpr (QSRC::kWaits) {
             // the wait for q is long: decode the cache bytes to bf16 and build
             // the RoPE tables before it, off the critical path
-            __syncthreads();   // lut
-            decode_all();
+            decode_k();
+            decode_v();
             rope_tables();
         }
         src.template fetch<QR, NR>(qo, ko, qa, qb, ka, kb);
@@ -318,37 +333,31 @@ __device__ __forceinline__ void attn_partial_body(AttnLds<RT, FUSED>& L, const Q
             }
         }
     }
-    // tokens m0..m0+MT-1 sit at positions base + m; those inside [0, max_pos) count
-    const int mv_lo = max(m0, -base);
-    const int mv_hi = min(min(M, m0 + MT) - 1, max_pos - 1 - base);
-    if (mv_hi < mv_lo || s0 > base + mv_hi) return;   // uniform: no token of this workgroup reaches the chunk
+    if constexpr (QSRC::kWaits)
+        if (idle) return;
     __syncthreads();
     if (FUSED && n_lo < n_hi) {
         // the step's rows in place of the cache bytes loaded above
         const int kr = s0 + wave * 16 + l16;
         if (kr >= n_lo && kr < n_hi) {
 #pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                kraw[kt] = *reinterpret_cast<const uint2*>(&knew[kr - s0][kt * 32 + lq * 8]);
-                if constexpr (QSRC::kWaits) kdec[kt] = kv8_bf16(lut, kraw[kt]);   // decoded ahead: again
-            }
+            for (int kt = 0; kt < 4; ++kt) kraw[kt] = *reinterpret_cast<const uint2*>(&knew[kr - s0][kt * 32 + lq * 8]);
         }
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
-                bool changed = false;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const int vr = s0 + kt * 32 + lq * 8 + t;
-                    if (vr >= n_lo && vr < n_hi) {
-                        vraw[c][kt][t] = vnew[vr - s0][wave * 32 + l16 + c * 16];
-                        changed = true;
-                    }
-                }
-                if constexpr (QSRC::kWaits)
-                    if (changed) vdec[kt][c] = decode_v(kt, c);
+            for (int t = 0; t < 8; ++t) {
+                const int vr = s0 + kt * 32 + lq * 8 + t;
+                if (vr >= n_lo && vr < n_hi) vraw[kt][t] = *reinterpret_cast<const uint16_t*>(&vnew[vr - s0][wave * 32 + 2 * l16]);
             }
+        if constexpr (QSRC::kWaits) {   // decoded ahead: again
+            decode_k();
+            decode_v();
+        }
+    }
+    if constexpr (!QSRC::kWaits) {
+        decode_k();
+        decode_v();
     }
     // ---- 2. scores, wave = positions 16*wave + l16
     mx::v4f sacc[RT];
@@ -356,12 +365,9 @@ __device__ __forceinline__ void attn_partial_body(AttnLds<RT, FUSED>& L, const Q
     for (int rt = 0; rt < RT; ++rt) sacc[rt] = mx::v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-        uint4 kb;
-        if constexpr (QSRC::kWaits) kb = kdec[kt];
-        else kb = kv8_bf16(lut, kraw[kt]);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
-            sacc[rt] = mfma_bf16(*reinterpret_cast<const uint4*>(&qs[rt * 16 + l16][kt * 32 + lq * 8]), kb, sacc[rt]);
+            sacc[rt] = mfma_bf16(*reinterpret_cast<const uint4*>(&qs[rt * 16 + l16][kt * 32 + lq * 8]), kdec[kt], sacc[rt]);
     }
     // ---- 3. softmax statistics
     const int s = s0 + wave * 16 + l16;
@@ -396,26 +402,20 @@ __device__ __forceinline__ void attn_partial_body(AttnLds<RT, FUSED>& L, const Q
         }
     __syncthreads();
     if (tid < R) rstat[1][tid] = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
-    // ---- 4. O = P V, wave = columns 32*wave + 16c + l16
+    // ---- 4. O = P V, wave = columns 32*wave + 2 l16 + c
     mx::v4f oacc[RT][2];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) oacc[rt][0] = oacc[rt][1] = mx::v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
-        uint4 vb[2];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            if constexpr (QSRC::kWaits) vb[c] = vdec[kt][c];
-            else vb[c] = decode_v(kt, c);
-        }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const uint4 ah = *reinterpret_cast<const uint4*>(&phi[rt * 16 + l16][kt * 32 + lq * 8]);
             const uint4 al = *reinterpret_cast<const uint4*>(&plo[rt * 16 + l16][kt * 32 + lq * 8]);
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
-                oacc[rt][c] = mfma_bf16(ah, vb[c], oacc[rt][c]);
-                oacc[rt][c] = mfma_bf16(al, vb[c], oacc[rt][c]);
+                oacc[rt][c] = mfma_bf16(ah, vdec[kt][c], oacc[rt][c]);
+                oacc[rt][c] = mfma_bf16(al, vdec[kt][c], oacc[rt][c]);
             }
         }
     }
@@ -428,8 +428,7 @@ __device__ __forceinline__ void attn_partial_body(AttnLds<RT, FUSED>& L, const Q
             const int m = m0 + r / G;
             if (m < mv_lo || m > mv_hi || s0 > base + m) continue;   // no record: the merge reads chunks up to the token's position
             float* rec = part + (((int64_t)m * Hq + g * G + r % G) * nchunk + chunk) * kPart;
-#pragma unroll
-            for (int c = 0; c < 2; ++c) rec[4 + wave * 32 + c * 16 + l16] = oacc[rt][c][i];
+            *reinterpret_cast<float2*>(rec + 4 + wave * 32 + 2 * l16) = make_float2(oacc[rt][0][i], oacc[rt][1][i]);
             if (wave == 0 && l16 == 0) {
                 rec[0] = rstat[0][r];
                 rec[1] = rstat[1][r];

@@ -63,7 +63,7 @@ constexpr int kLdsRow = kD + 8;
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+using kv::f16x2_t;
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
@@ -82,49 +82,6 @@ __device__ __forceinline__ int units_per_split(int n, int nsplit) {
     const int nu = (n + kUnit - 1) / kUnit;
     const int per = (nu + nsplit - 1) / nsplit;
     return max(4, (per + 3) & ~3);
-}
-
-// Four codec bytes as OCP E4M3 bytes of the same values; bit 7 of a byte of
-// `e15` is set when that byte's exponent field is 15 (then the result is not
-// used).
-__device__ __forceinline__ uint32_t codec_to_ocp(uint32_t w, uint32_t& e15) {
-    const uint32_t ex = w & 0x78787878u;
-    const uint32_t nz = (ex + 0x78787878u) & 0x80808080u;    // exponent not 0
-    e15 |= ex + 0x08080808u;
-    const uint32_t keep = 0x80808080u | (nz - (nz >> 7));    // the byte, or its sign only
-    const uint32_t sub = __builtin_amdgcn_perm(0x1E1C1A18u, 0x14100800u, w & 0x07070707u);   // m * 2^-6 as a normal code
-    return (w & keep) | (sub & ~keep);
-}
-
-// Bytes 2 HI, 2 HI + 1 of w as two bf16 (K) or fp16 (V).  EXP15: the bytes
-// whose bit 7 is set in f had exponent 15 and are in w with exponent 14; the
-// codec reads them as 56 (8 + m), 3.5 times that (exact in both).
-template <bool HI, bool F16, bool EXP15>
-__device__ __forceinline__ uint32_t pair_of(uint32_t w, uint32_t f) {
-    if constexpr (F16) {
-        const f16x2_t r = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, HI);
-        if constexpr (!EXP15) return __builtin_bit_cast(uint32_t, r);
-        const f16x2_t k = {(_Float16)(f & (HI ? 0x800000u : 0x80u) ? 3.5f : 1.0f),
-                           (_Float16)(f & (HI ? 0x80000000u : 0x8000u) ? 3.5f : 1.0f)};
-        return __builtin_bit_cast(uint32_t, r * k);
-    } else {
-        const uint32_t r = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI));
-        if constexpr (!EXP15) return r;
-        const float a = __uint_as_float(r << 16) * (f & (HI ? 0x800000u : 0x80u) ? 3.5f : 1.0f);
-        const float b = __uint_as_float(r & 0xFFFF0000u) * (f & (HI ? 0x80000000u : 0x8000u) ? 3.5f : 1.0f);
-        return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xFFFF0000u);
-    }
-}
-
-// A codec word ready for pair_of, and its exponent-15 flags.
-template <bool EXP15>
-__device__ __forceinline__ uint32_t ready(uint32_t w, uint32_t& f, uint32_t& e15) {
-    f = 0;
-    if constexpr (EXP15) {
-        f = ((w & 0x78787878u) + 0x08080808u) & 0x80808080u;
-        w -= f >> 4;
-    }
-    return codec_to_ocp(w, e15);
 }
 
 // A unit's bytes as a lane loads them, by buffer loads relative to the
@@ -160,9 +117,9 @@ __device__ __forceinline__ void decode_k(const RawK& r, uint4 (&kd)[2][4], uint3
             uint32_t w[4], f[4], o[8];
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
-                w[d] = ready<EXP15>(r.k[t][j][d], f[d], e15);
-                o[2 * d] = pair_of<false, false, EXP15>(w[d], f[d]);
-                o[2 * d + 1] = pair_of<true, false, EXP15>(w[d], f[d]);
+                w[d] = kv::ready<EXP15>(r.k[t][j][d], f[d], e15);
+                o[2 * d] = kv::pair_of<false, false, EXP15>(w[d], f[d]);
+                o[2 * d + 1] = kv::pair_of<true, false, EXP15>(w[d], f[d]);
             }
             kd[t][2 * j] = make_uint4(o[0], o[1], o[2], o[3]);
             kd[t][2 * j + 1] = make_uint4(o[4], o[5], o[6], o[7]);
@@ -176,17 +133,17 @@ __device__ __forceinline__ void decode_v(const RawV& r, uint4 (&vd)[8], uint32_t
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
             uint32_t fa, fb;
-            const uint32_t a = ready<EXP15>(r.v[2 * t2][d], fa, e15), b = ready<EXP15>(r.v[2 * t2 + 1][d], fb, e15);
+            const uint32_t a = kv::ready<EXP15>(r.v[2 * t2][d], fa, e15), b = kv::ready<EXP15>(r.v[2 * t2 + 1][d], fb, e15);
             const uint32_t c01 = __builtin_amdgcn_perm(b, a, 0x05010400u), c23 = __builtin_amdgcn_perm(b, a, 0x07030602u);
             uint32_t f01 = 0, f23 = 0;
             if constexpr (EXP15) {
                 f01 = __builtin_amdgcn_perm(fb, fa, 0x05010400u);
                 f23 = __builtin_amdgcn_perm(fb, fa, 0x07030602u);
             }
-            o[4 * d][t2] = pair_of<false, true, EXP15>(c01, f01);
-            o[4 * d + 1][t2] = pair_of<true, true, EXP15>(c01, f01);
-            o[4 * d + 2][t2] = pair_of<false, true, EXP15>(c23, f23);
-            o[4 * d + 3][t2] = pair_of<true, true, EXP15>(c23, f23);
+            o[4 * d][t2] = kv::pair_of<false, true, EXP15>(c01, f01);
+            o[4 * d + 1][t2] = kv::pair_of<true, true, EXP15>(c01, f01);
+            o[4 * d + 2][t2] = kv::pair_of<false, true, EXP15>(c23, f23);
+            o[4 * d + 3][t2] = kv::pair_of<true, true, EXP15>(c23, f23);
         }
     }
 #pragma unroll

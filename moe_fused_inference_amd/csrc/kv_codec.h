@@ -72,4 +72,50 @@ __device__ __forceinline__ uint32_t e4m3_encode(float v, int codec) {
     return codec ? e4m3_torch_encode(v) : e4m3_ref_encode(v);
 }
 
+// ---- many bytes at a time, by the hardware's OCP E4M3 conversion
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+
+// Four codec bytes as OCP E4M3 bytes of the same values; bit 7 of a byte of
+// `e15` is set when that byte's exponent field is 15 (then the result is not
+// used).
+__device__ __forceinline__ uint32_t codec_to_ocp(uint32_t w, uint32_t& e15) {
+    const uint32_t ex = w & 0x78787878u;
+    const uint32_t nz = (ex + 0x78787878u) & 0x80808080u;    // exponent not 0
+    e15 |= ex + 0x08080808u;
+    const uint32_t keep = 0x80808080u | (nz - (nz >> 7));    // the byte, or its sign only
+    const uint32_t sub = __builtin_amdgcn_perm(0x1E1C1A18u, 0x14100800u, w & 0x07070707u);   // m * 2^-6 as a normal code
+    return (w & keep) | (sub & ~keep);
+}
+
+// Bytes 2 HI, 2 HI + 1 of w as two bf16 (K) or fp16 (V).  EXP15: the bytes
+// whose bit 7 is set in f had exponent 15 and are in w with exponent 14; the
+// codec reads them as 56 (8 + m), 3.5 times that (exact in both).
+template <bool HI, bool F16, bool EXP15>
+__device__ __forceinline__ uint32_t pair_of(uint32_t w, uint32_t f) {
+    if constexpr (F16) {
+        const f16x2_t r = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, HI);
+        if constexpr (!EXP15) return __builtin_bit_cast(uint32_t, r);
+        const f16x2_t k = {(_Float16)(f & (HI ? 0x800000u : 0x80u) ? 3.5f : 1.0f),
+                           (_Float16)(f & (HI ? 0x80000000u : 0x8000u) ? 3.5f : 1.0f)};
+        return __builtin_bit_cast(uint32_t, r * k);
+    } else {
+        const uint32_t r = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI));
+        if constexpr (!EXP15) return r;
+        const float a = __uint_as_float(r << 16) * (f & (HI ? 0x800000u : 0x80u) ? 3.5f : 1.0f);
+        const float b = __uint_as_float(r & 0xFFFF0000u) * (f & (HI ? 0x80000000u : 0x8000u) ? 3.5f : 1.0f);
+        return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xFFFF0000u);
+    }
+}
+
+// A codec word ready for pair_of, and its exponent-15 flags.
+template <bool EXP15>
+__device__ __forceinline__ uint32_t ready(uint32_t w, uint32_t& f, uint32_t& e15) {
+    f = 0;
+    if constexpr (EXP15) {
+        f = ((w & 0x78787878u) + 0x08080808u) & 0x80808080u;
+        w -= f >> 4;
+    }
+    return codec_to_ocp(w, e15);
+}
+
 }  // namespace kv

@@ -225,3 +225,19 @@ def test_attn_decode_fused_split_matches_two_ops(codec):
     equals qk_norm_rope_kv followed by attn_decode_mx bit for bit."""
     from tests.test_gpu_decode_step import test_attn_decode_fused_matches_two_ops as check
     check(5, 32, 4, 6001, 5998, codec)
+
+
+@pytest.mark.parametrize("M,Hq,Hkv,max_pos,base", [(1, 32, 4, 300, 290), (5, 8, 8, 200, 190)])
+def test_attn_decode_chunks_every_byte(dext, M, Hq, Hkv, max_pos, base):
+    """The chunk pass over caches that hold every codec byte, exponent fields 0
+    and 15 among them."""
+    rng = np.random.default_rng(M + Hq)
+    kvk_np = rng.integers(0, 256, size=(max_pos, Hkv, 128), dtype=np.uint8)
+    kvv_np = rng.integers(0, 256, size=(max_pos, Hkv, 128), dtype=np.uint8)
+    q = _bf16(rng.standard_normal((M, Hq, 128)) * 1e-3)      # scores of order one
+    sc = torch.empty((M, Hq, max_pos), dtype=torch.float32, device=DEV)
+    o = dext.attn_decode(q.to(DEV), torch.from_numpy(kvk_np).to(DEV), torch.from_numpy(kvv_np).to(DEV),
+                         torch.tensor([base], dtype=torch.int32, device=DEV), sc, M)
+    torch.cuda.synchronize()
+    ref, _ = attn.attn_decode_ref(q.float().numpy(), kvk_np, kvv_np, base)
+    assert_close(np_(o), ref, what=f"every cache byte, M={M}")
