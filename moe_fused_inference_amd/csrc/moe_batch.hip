@@ -154,7 +154,6 @@ __host__ __device__ constexpr int gu_lds_bytes(int H) { return gu_sb_off(H) + 4 
 template <bool STAGED>
 __global__ __launch_bounds__(256) void batch_gateup_kernel(BatchArgs a) {
     __shared__ int s_slot[kMaxTok];
-    __shared__ int s_cnt, s_own;
     __shared__ float gu[2][kMaxTok][33];
     const int rb = blockIdx.x, s = blockIdx.y;
     const int S = a.M * a.E;
@@ -166,39 +165,37 @@ __global__ __launch_bounds__(256) void batch_gateup_kernel(BatchArgs a) {
         for (int i = rb * per + tid; i < min(n, (rb + 1) * per); i += 256) a.y[i] = 0.0f;
     }
     // ---- the first slot naming expert e owns it and gathers its tokens: all
-    // S <= 128 ids in one round of loads (two per lane), then ballots
-    if (wave == 0) {
-        const int v0 = lane < S ? a.ids[lane] : -1;
-        const int v1 = 64 + lane < S ? a.ids[64 + lane] : -1;
-        const bool any = __ballot((lane < s && v0 == e) || (64 + lane < s && v1 == e)) != 0ull;
-        const unsigned long long b0 = __ballot(lane >= s && lane < S && v0 == e);
-        const unsigned long long b1 = __ballot(64 + lane >= s && 64 + lane < S && v1 == e);
-        const unsigned long long below = (1ull << lane) - 1ull;
-        if (!any) {
-            const int p0 = __popcll(b0 & below), p1 = __popcll(b0) + __popcll(b1 & below);
-            if (((b0 >> lane) & 1ull) && p0 < kMaxTok) s_slot[p0] = lane;
-            if (((b1 >> lane) & 1ull) && p1 < kMaxTok) s_slot[p1] = 64 + lane;
-        }
-        if (lane == 0) {
-            const int cnt = __popcll(b0) + __popcll(b1);
-            s_own = any ? 0 : 1;
-            s_cnt = cnt < kMaxTok ? cnt : kMaxTok;
-        }
-    }
-    __syncthreads();
+    // S <= 128 ids in one round of loads (two per lane), then ballots.  Every
+    // wave does this for itself (and writes the same list), so its weights are
+    // under way one memory latency after the start, with no barrier before them.
+    const int v0 = lane < S ? a.ids[lane] : -1;
+    const int v1 = 64 + lane < S ? a.ids[64 + lane] : -1;
+    const bool own = __ballot((lane < s && v0 == e) || (64 + lane < s && v1 == e)) == 0ull;
+    const unsigned long long b0 = __ballot(lane >= s && lane < S && v0 == e);
+    const unsigned long long b1 = __ballot(64 + lane >= s && 64 + lane < S && v1 == e);
+    const int cnt = min(__popcll(b0) + __popcll(b1), kMaxTok);
     const bool valid_e = e >= 0 && e < a.n_experts;   // other ids contribute h = 0
     // the owner table of the down launch: slot s owns a valid expert (first
     // slot naming it), its member count and member slots (token order)
-    if (rb == 0 && wave == 0) {
-        const int S_ = a.M * a.E;
-        if (lane == 0) {
-            a.meta[s] = (uint8_t)(s_own && valid_e ? 1 : 0);
-            a.meta[S_ + s] = (uint8_t)(s_own ? s_cnt : 0);
-        }
-        if (s_own && lane < s_cnt) a.meta[2 * S_ + s * kMaxTok + lane] = (uint8_t)s_slot[lane];
+    if (rb == 0 && tid == 0) {
+        a.meta[s] = (uint8_t)(own && valid_e ? 1 : 0);
+        a.meta[S + s] = (uint8_t)(own ? cnt : 0);
     }
-    if (!s_own) return;
-    const int cnt = s_cnt;
+    if (!own) return;   // uniform
+    {
+        const unsigned long long below = (1ull << lane) - 1ull;
+        const int p0 = __popcll(b0 & below), p1 = __popcll(b0) + __popcll(b1 & below);
+        const bool i0 = ((b0 >> lane) & 1ull) && p0 < kMaxTok, i1 = ((b1 >> lane) & 1ull) && p1 < kMaxTok;
+        if (i0) s_slot[p0] = lane;
+        if (i1) s_slot[p1] = 64 + lane;
+        if (rb == 0 && wave == 0) {
+            uint8_t* ms = a.meta + 2 * S + s * kMaxTok;
+            if (i0) ms[p0] = (uint8_t)lane;
+            if (i1) ms[p1] = (uint8_t)(64 + lane);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the wave's own list is written
+    __builtin_amdgcn_wave_barrier();
     const int l16 = lane & 15, q = lane >> 4;
     const int H = a.H, Mi = a.Mi;
     const int proj = wave >> 1;
@@ -212,6 +209,11 @@ __global__ __launch_bounds__(256) void batch_gateup_kernel(BatchArgs a) {
     if constexpr (STAGED) {
         extern __shared__ __align__(16) uint8_t dyn[];
         const int steps = nch / 4;
+        // every K step of the wave's weight rows in flight
+        uint4 bq[kGuMaxSteps];
+#pragma unroll
+        for (int st = 0; st < kGuMaxSteps; ++st)
+            if (st < steps) bq[st] = *reinterpret_cast<const uint4*>(wrow + 16 * (4 * st + q));
         const uint32_t lds0 = mx::lds_addr(dyn);
         // member rows of x (wave w: members w, w + 4, ...) at t * gu_arow(H)
         const mx::v4u rx = mx::buf_rsrc(a.xq, (int64_t)a.M * (H / 2));
@@ -234,11 +236,6 @@ __global__ __launch_bounds__(256) void batch_gateup_kernel(BatchArgs a) {
         for (int c = 0; c * 1024 < 16 * nch; ++c)
             if (c * 1024 + 16 * lane < 16 * nch)
                 mx::dma16(16u * lane, rbs, (uint32_t)(c * 1024), lds0 + gu_sb_off(H) + wave * 16 * nch + c * 1024);
-        // every K step of the wave's weight rows in flight
-        uint4 bq[kGuMaxSteps];
-#pragma unroll
-        for (int st = 0; st < kGuMaxSteps; ++st)
-            if (st < steps) bq[st] = *reinterpret_cast<const uint4*>(wrow + 16 * (4 * st + q));
         // all of it has landed (the copies of every wave, at the barrier)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
@@ -434,6 +431,11 @@ __global__ __launch_bounds__(64 * kDownWaves) void batch_down_lds_kernel(BatchAr
     const uint8_t* mcnt = a.meta + S;
     const uint8_t* mslots = a.meta + 2 * S;
     const bool o0 = lane < S && own[lane] != 0, o1 = 64 + lane < S && own[64 + lane] != 0;
+    // slot lane's and slot 64 + lane's expert and member count, for readlane: a
+    // load per owner would be a second latency before its weights
+    const int e0 = lane < S ? a.ids[lane] : 0, e1 = 64 + lane < S ? a.ids[64 + lane] : 0;
+    const int c0 = lane < S ? (int)mcnt[lane] : 0, c1 = 64 + lane < S ? (int)mcnt[64 + lane] : 0;
+    auto of_slot = [](int lo, int hi, int sl) { return __builtin_amdgcn_readlane(sl < 64 ? lo : hi, sl & 63); };
     const uint64_t mlo = __ballot(o0), mhi = __ballot(o1);
     const int nown = __popcll(mlo) + __popcll(mhi);
     if (tid < S) s_w[tid] = a.w[tid];
@@ -451,16 +453,15 @@ __global__ __launch_bounds__(64 * kDownWaves) void batch_down_lds_kernel(BatchAr
     bool first = true;
     // wave w of half h: owners 2 w + h, 2 (w + kDownWaves) + h, ... in rounds of OPR
     for (int k0 = 2 * wave + half; first || k0 < nown; k0 += 2 * kDownWaves * OPR) {
-        int oslot[OPR], oe[OPR], ocnt[OPR], mv[OPR];
+        int oslot[OPR], ocnt[OPR], mv[OPR];
         uint4 bq[OPR][MS];
 #pragma unroll
         for (int o = 0; o < OPR; ++o) {
             const int k = k0 + 2 * kDownWaves * o;
             oslot[o] = k < nown ? nth_set(mlo, mhi, k) : -1;
             const int sl = oslot[o] < 0 ? 0 : oslot[o];
-            const int e = oslot[o] < 0 ? 0 : a.ids[sl];
-            oe[o] = e;
-            ocnt[o] = oslot[o] < 0 ? 0 : (int)mcnt[sl];
+            const int e = oslot[o] < 0 ? 0 : of_slot(e0, e1, sl);
+            ocnt[o] = oslot[o] < 0 ? 0 : of_slot(c0, c1, sl);
             mv[o] = lane < ocnt[o] ? (int)mslots[sl * kMaxTok + lane] : 0;   // written to LDS after the wait
             // the owner's down rows for the 16 columns (zero-extent for no owner) and their scales
             const uint8_t* wrow = a.dwp + ((int64_t)e * H + cb * 16) * (Mi / 2);
