@@ -212,3 +212,38 @@ def test_moe_compute_routing_sizes(dext, T, k, n_exp):
     torch.cuda.synchronize()
     used = [e for e in range(n_exp) if bool((ti == e).any())]
     check_prefill(out, x, ti, tv, oracle_experts(stack, used), f"routing T={T} k={k} n={n_exp}")
+
+
+# the gate/up epilogue's packed fp16 quantizer: every midpoint of E2M1, either sign, and a NaN, which counts as 0
+@pytest.mark.parametrize("H,Mi", [(256, 256), (64, 32)])
+def test_moe_compute_h_midpoints_and_nan(dext, H, Mi):
+    """h = 128 u exactly (silu(128) = 128), u = x0 w0 + x1 w1 on the midpoints
+    of a block whose largest magnitude is 6 steps: the codes round up in
+    magnitude, and a down projection that copies h shows them exactly.  With
+    NaN scales on a gate row the feature is as if its weights were zero."""
+    pairs = [(0, .5), (.5, .5), (1, .5), (1.5, .5), (2, 1), (3, 1), (4, 2), (6, 0)]   # w0 + w1 / 2 = the midpoints, 6
+    codes = [.5, 1, 1.5, 2, 3, 4, 6, 6]
+    gate, up, down = torch.zeros(Mi, H), torch.zeros(Mi, H), torch.zeros(H, Mi)
+    gate[:, 0] = 2.0
+    want = torch.zeros(H)
+    for f in range(32):
+        sign = -1.0 if f & 8 else 1.0
+        if f >= 16:
+            continue   # zeros: code 0
+        up[f, 0], up[f, 1] = sign * pairs[f % 8][0], sign * pairs[f % 8][1]
+        down[f, f] = 1.0
+        want[f] = sign * codes[f % 8] * 8192.0
+    x = torch.zeros(5, H, device=DEV, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1] = 64.0, 32.0
+    parts = {}
+    for nm, w in (("gate", gate), ("up", up), ("down", down)):
+        q, s = dext.prequant(w.to(DEV).bfloat16())
+        parts[nm + "_wp"], parts[nm + "_ws"] = q[None].contiguous(), s[None].contiguous()
+    ti = torch.zeros((5, 1), dtype=torch.int64, device=DEV)
+    tv = torch.ones((5, 1), device=DEV).bfloat16()
+    out = moe_layer.moe_compute(x, ti, tv, moe_layer.StackedExperts(**parts))
+    assert torch.equal(out.float().cpu(), want.expand(5, H))
+    parts["gate_ws"][0, 4] = 255
+    want[4] = 0.0
+    out = moe_layer.moe_compute(x, ti, tv, moe_layer.StackedExperts(**parts))
+    assert torch.equal(out.float().cpu(), want.expand(5, H))
