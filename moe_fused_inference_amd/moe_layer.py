@@ -523,7 +523,7 @@ def moe_compute(h, topi, scores, experts, out=None, ws=None):
     (runtime/model_runner_v2.py:108-122): h (T, H) bf16, topi (T, k) int64,
     scores (T, k) (used as bf16, as moe_route returns them), experts either a
     StackedExperts or the reference's dict of per-expert spec dicts.  Returns
-    the bf16 (T, H) MoE output.  Five launches, no host synchronisation (the
+    the bf16 (T, H) MoE output.  Five launches (four up to 4096 pairs), no host synchronisation (the
     dict form builds a small pointer table first)."""
     lib = _lib.load()
     if h.dim() != 2 or h.dtype != torch.bfloat16 or not h.is_cuda:
