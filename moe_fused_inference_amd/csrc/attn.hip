@@ -130,8 +130,10 @@ int launch_attn(const void* q, const uint8_t* kvk, const uint8_t* kvv, const int
     // whose records the layer launch merges, and so does a short cache, where
     // both wait on latency: 4096 positions, 1 token 9.8 against 8.4 us, 9 tokens
     // 19.6 against 15.4; 23001 positions, 4 tokens 29.5 against 19.2, 9 tokens
-    // 54.4 against 25.2, 16 tokens 73.6 against 34.0.
-    if (M > 1 && max_pos > 64 * kChunk && merge && G <= 16 && (G & (G - 1)) == 0) {
+    // 54.4 against 25.2, 16 tokens 73.6 against 34.0.  (It addresses a cache
+    // with 31-bit offsets.)
+    if (M > 1 && max_pos > 64 * kChunk && merge && G <= 16 && (G & (G - 1)) == 0 &&
+        (int64_t)max_pos * Hkv * kD < (1ll << 31)) {
         if constexpr (FUSED) {
             // the head norm, RoPE and KV write as their own launch, q past the records
             void* qb = static_cast<uint8_t*>(workspace) + mxh::attn_split_record_bytes(M, Hq, Hkv, max_pos);

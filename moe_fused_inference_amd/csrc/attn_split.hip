@@ -57,7 +57,7 @@ using am::kD;
 using am::kPart;
 
 constexpr int kUnit = 32;      // positions per wave and step
-constexpr float kSlack = 8.0f;
+constexpr float kSlack = 8.0f, kHead = 7.0f;   // a term is at most 2^15 (fp16: 65504)
 constexpr int kMaxRT = 3;      // 16-row tiles per workgroup
 constexpr int kLdsRow = kD + 8;
 
@@ -319,9 +319,12 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(SplitArgs a) {
             mx_ = max_over_lq(mx_) * a.c;
             // m is the reference of the row's terms, not their maximum: it follows
             // the maximum only past a factor of 2^kSlack (any reference gives the
-            // same quotient; the sums of a first unit need no rescaling at all)
-            if (__ballot(mx_ > m[rt] + kSlack)) {
-                const float mn = fmaxf(m[rt], mx_);
+            // same quotient; the sums of a first unit need no rescaling at all).
+            // It stays 2^kHead below it, so that what fp16 cuts off a term
+            // (2^-24) is 2^-31 of the largest: a row with one large score and
+            // thousands of small ones keeps the small ones' sum
+            if (__ballot(mx_ > m[rt] + (kHead + kSlack))) {
+                const float mn = fmaxf(m[rt], mx_ - kHead);
                 if (u != u0 + wave) {
                     const float al = __builtin_amdgcn_exp2f(m[rt] - (mn == -INFINITY ? 0.0f : mn));
                     l[rt] *= al;

@@ -219,6 +219,28 @@ def test_attn_decode_split_vs_oracle(dext, M, Hq, Hkv, max_pos, base):
     assert torch.isnan(sc[live[0], :, base + live[0] + 1:]).all()
 
 
+def test_attn_decode_split_one_large_score(dext):
+    """A position that takes most of the weight leaves the sum of the many small
+    ones: scores of s at position 0 and 0 elsewhere, values 1 and 16."""
+    M, Hq, Hkv, max_pos, base = 16, 32, 2, 65536, 65515
+    kvk = torch.zeros((max_pos, Hkv * 128), dtype=torch.uint8, device=DEV)
+    kvv = torch.full_like(kvk, 0x58)                                     # 16
+    kvk[0], kvv[0] = 0x38, 0x38                                          # 1
+    q = torch.full((M, Hq, 128), 1.546875, dtype=torch.bfloat16, device=DEV)
+    o = dext.attn_decode(q, kvk.view(max_pos, Hkv, 128), kvv.view(max_pos, Hkv, 128),
+                         torch.tensor([base], dtype=torch.int32, device=DEV),
+                         torch.empty((M, Hq, max_pos), dtype=torch.float32, device=DEV), M)
+    torch.cuda.synchronize()
+    w = np.exp(-1.546875 * 128 / np.sqrt(128.0))                         # 2^-25.2
+    n = base + np.arange(M, dtype=np.float64)
+    ref = ((1 + 16 * w * n) / (1 + w * n))[:, None, None]
+    # 2^-31 of the largest term lost on each of the 416 positions it shares a
+    # wave with, times 16: 3e-6; the wave's 26 matrix instructions add to a sum
+    # of that term's size, up to 8 times each with 2^-23 cut off: 2.5e-5 (a
+    # reference at the row's maximum would lose 16 * 416 * 2^-25.2 = 1.7e-4)
+    assert np.abs(np_(o) / ref - 1).max() <= 3e-5
+
+
 @pytest.mark.parametrize("codec", [0, 1])
 def test_attn_decode_fused_split_matches_two_ops(codec):
     """Past 4096 positions mxfp4_attn_decode_fused with several tokens still
