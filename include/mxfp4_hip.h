@@ -171,8 +171,7 @@ int mxfp4_attn_decode_mx(const void* q, const uint8_t* kvk, const uint8_t* kvv, 
 
 /* mxfp4_attn_decode_fused: mxfp4_qk_norm_rope_kv followed by
  * mxfp4_attn_decode_mx in one pass over the cache (as those two for M > 1 and
- * max_pos > 4096, a cache under 2 GiB, G <= 16 a
- * power of two), bit-exact to that pair
+ * max_pos > 4096, G <= 16 a power of two), bit-exact to that pair
  * (same q, cache bytes, sc and outputs): qkv fp32 (M, (Hq + 2 Hkv) * D) are
  * the step's projections, the q heads are normalised and rotated inside the
  * attention kernel and the step's k / v rows (positions *dpos .. *dpos+M-1)

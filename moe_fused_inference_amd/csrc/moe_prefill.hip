@@ -525,6 +525,10 @@ __device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
 // on pairs, the amax as integers, which also shows a NaN, and one mixed fma a
 // feature for scale, tie and sign of zero.  MI355X, 2048 tokens x 8 of 128
 // experts, H = 2048, Mi = 768: the launch 63.1 -> 60.6 us.
+// (silu(g)*u is rounded to fp32 and then to fp16, as stated above; a lone
+// value's product and conversion had become one instruction that rounds the
+// product once, which is another fp16 value where the fp32 one is a midpoint:
+// 0 to 2 of the 12.6 million features then have another code or block scale.)
 template <int NI>
 __device__ __forceinline__ void gateup_epilogue(mx::v16f (&acc)[2][2], const GArgs& g, int n0, int off, int mt,
                                                 int mrows, int rbase, int wn, int lr, int h) {
