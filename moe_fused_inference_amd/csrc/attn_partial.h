@@ -53,8 +53,8 @@ template <bool EXP15>
 __device__ __forceinline__ uint4 kv8_bf16(uint2 w, uint32_t& e15) {
     uint32_t f0, f1;
     const uint32_t a = kv::ready<EXP15>(w.x, f0, e15), b = kv::ready<EXP15>(w.y, f1, e15);
-    return make_uint4(kv::pair_of<false, false, EXP15>(a, f0), kv::pair_of<true, false, EXP15>(a, f0),
-                      kv::pair_of<false, false, EXP15>(b, f1), kv::pair_of<true, false, EXP15>(b, f1));
+    return make_uint4(kv::pair_of<false, EXP15>(a, f0), kv::pair_of<true, EXP15>(a, f0),
+                      kv::pair_of<false, EXP15>(b, f1), kv::pair_of<true, EXP15>(b, f1));
 }
 
 // The chunk pass's LDS.
@@ -190,8 +190,8 @@ __device__ __forceinline__ void attn_partial_body(AttnLds<RT, FUSED>& L, const Q
             for (int t = 0; t < 4; ++t) {
                 uint32_t f;
                 const uint32_t w = kv::ready<E>(__builtin_amdgcn_perm(vraw[kt][2 * t + 1], vraw[kt][2 * t], 0x05010400u), f, e15);
-                o[0][t] = kv::pair_of<false, false, E>(w, f);
-                o[1][t] = kv::pair_of<true, false, E>(w, f);
+                o[0][t] = kv::pair_of<false, E>(w, f);
+                o[1][t] = kv::pair_of<true, E>(w, f);
             }
 #pragma unroll
             for (int c = 0; c < 2; ++c) vdec[kt][c] = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);

@@ -6,8 +6,8 @@
 //                      positions against up to 48 query rows (tokens x heads
 //                      of the kv head), a wave taking every fourth unit of 32
 //                      positions with its own running softmax; the four
-//                      waves' sums meet in LDS -> one record (max, sum, 128
-//                      column sums) per query row and split.
+//                      waves' sums meet in LDS -> one record (reference, sum,
+//                      128 column sums) per query row and split.
 //   attn_split_merge_kernel  workgroup (query head, token): merges the row's
 //                      records (am::merge_head) to o and / or its MXFP4 rows.
 //
@@ -32,19 +32,22 @@
 //    3 instructions a byte and no LDS table.  Bytes of exponent 15, which the
 //    codec reads as 56 (8 + m) and a cache holds only for |v| >= 240, send the
 //    wave's unit through a longer path.
-//  * P and V are fp16 in the second product (every codec value is exact in
-//    fp16 too) and P is split into a high and a low part (two MFMAs), which
-//    keeps 21 bits of a term; exp is the hardware's exp2 of fma(s, log2(e) /
-//    sqrt(D), -m), with m kept in that base so that a row's terms and the merge
-//    agree on it.
+//  * In the second product V is bf16 (every codec value is) and P is three bf16
+//    parts, whose sum is the fp32 probability at any size: one score far above
+//    the others leaves the others' sum.  (Two fp16 parts, a third of the MFMAs
+//    and a few conversions less, took 134 us of the 136 below, but cut a
+//    probability off at 2^-31 of its row's largest: 65520 scores e^17.5 below
+//    one, of values 448 and 2^-6, were wrong by 1e-4, and are by 7e-7.)  exp is
+//    the hardware's exp2 of fma(s, log2(e) / sqrt(D), -m), with m kept in that
+//    base so that a row's terms and the merge agree on it.
 //  * At most three row tiles a workgroup: their accumulators, a unit's operands
 //    and the next unit's bytes fit 256 registers, two waves per SIMD.  (Five
 //    tiles decode each byte once for 72 rows, but past 256 registers the
 //    accumulators move between register files at every step: 37 us against 25
 //    at 9 tokens and 23001 positions.)
-// Measured on MI355X (32 / 4 heads, both launches, the raw scores kept): 9
-// tokens over 23001 positions 54.4 us by chunks, 25.2 here (50 MB of cache and
-// scores: 2.0 TB/s); relative error against 64 bits 1.9e-6 and 2.4e-7.
+// Measured on MI355X (32 / 4 heads, the raw scores kept, four layers, each with
+// its KV write, in a graph): 9 tokens over 23001 positions 243 us by chunks, 136
+// here; relative error against 64 bits 1.9e-6 and 2.1e-7.
 #include "attn_merge.h"
 #include "attn_split.h"
 #include "kv_codec.h"
@@ -57,24 +60,19 @@ using am::kD;
 using am::kPart;
 
 constexpr int kUnit = 32;      // positions per wave and step
-constexpr float kSlack = 8.0f, kHead = 7.0f;   // a term is at most 2^15 (fp16: 65504)
+constexpr float kSlack = 8.0f;         // a term is at most 2^8
+constexpr float kWide = 262144.0f;     // a reference past it: an exponent's rounding is up to 2^-6 and more
+constexpr float kNone = -3e38f;        // the reference of a row that has seen nothing: exp2(-inf - kNone) = 0
 constexpr int kMaxRT = 3;      // 16-row tiles per workgroup
 constexpr int kLdsRow = kD + 8;
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-using kv::f16x2_t;
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ mx::v4f mfma_bf16(uint4 a, uint4 b, mx::v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
                                                    0, 0, 0);
-}
-
-__device__ __forceinline__ mx::v4f mfma_f16(uint4 a, uint4 b, mx::v4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
-                                                  0, 0);
 }
 
 // Units per split for a context of n positions: equal shares in whole rounds of the four waves.
@@ -118,12 +116,20 @@ __device__ __forceinline__ void decode_k(const RawK& r, uint4 (&kd)[2][4], uint3
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
                 w[d] = kv::ready<EXP15>(r.k[t][j][d], f[d], e15);
-                o[2 * d] = kv::pair_of<false, false, EXP15>(w[d], f[d]);
-                o[2 * d + 1] = kv::pair_of<true, false, EXP15>(w[d], f[d]);
+                o[2 * d] = kv::pair_of<false, EXP15>(w[d], f[d]);
+                o[2 * d + 1] = kv::pair_of<true, EXP15>(w[d], f[d]);
             }
             kd[t][2 * j] = make_uint4(o[0], o[1], o[2], o[3]);
             kd[t][2 * j + 1] = make_uint4(o[4], o[5], o[6], o[7]);
         }
+}
+__device__ __forceinline__ void decode_k(const RawK& r, uint4 (&kd)[2][4]) {
+    uint32_t e15 = 0;
+    decode_k<false>(r, kd, e15);
+    if (__ballot((e15 & 0x80808080u) != 0u)) {
+        uint32_t none = 0;
+        decode_k<true>(r, kd, none);
+    }
 }
 template <bool EXP15>
 __device__ __forceinline__ void decode_v(const RawV& r, uint4 (&vd)[8], uint32_t& e15) {
@@ -140,14 +146,47 @@ __device__ __forceinline__ void decode_v(const RawV& r, uint4 (&vd)[8], uint32_t
                 f01 = __builtin_amdgcn_perm(fb, fa, 0x05010400u);
                 f23 = __builtin_amdgcn_perm(fb, fa, 0x07030602u);
             }
-            o[4 * d][t2] = kv::pair_of<false, true, EXP15>(c01, f01);
-            o[4 * d + 1][t2] = kv::pair_of<true, true, EXP15>(c01, f01);
-            o[4 * d + 2][t2] = kv::pair_of<false, true, EXP15>(c23, f23);
-            o[4 * d + 3][t2] = kv::pair_of<true, true, EXP15>(c23, f23);
+            o[4 * d][t2] = kv::pair_of<false, EXP15>(c01, f01);
+            o[4 * d + 1][t2] = kv::pair_of<true, EXP15>(c01, f01);
+            o[4 * d + 2][t2] = kv::pair_of<false, EXP15>(c23, f23);
+            o[4 * d + 3][t2] = kv::pair_of<true, EXP15>(c23, f23);
         }
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) vd[c] = make_uint4(o[c][0], o[c][1], o[c][2], o[c][3]);
+}
+__device__ __forceinline__ void decode_v(const RawV& r, uint4 (&vd)[8]) {
+    uint32_t e15 = 0;
+    decode_v<false>(r, vd, e15);
+    if (__ballot((e15 & 0x80808080u) != 0u)) {
+        uint32_t none = 0;
+        decode_v<true>(r, vd, none);
+    }
+}
+
+// Eight fp32 terms as three bf16 parts each, whose sum each is (8 bits a part,
+// rounded to nearest, the rest exact).
+__device__ __forceinline__ void parts(float (&t)[8], uint4 (&p)[3]) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{t[2 * i], t[2 * i + 1]}), bf16x2_t));
+            t[2 * i] -= __uint_as_float(o[i] << 16);
+            t[2 * i + 1] -= __uint_as_float(o[i] & 0xFFFF0000u);
+        }
+        p[j] = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+
+// a * b rounded, minus c: not one fma.
+__device__ __forceinline__ float mul_then_sub(float a, float b, float c) {
+#pragma clang fp contract(off)
+    const float ab = a * b;
+    return ab - c;
 }
 
 // The maximum over the four lanes l, l ^ 16, l ^ 32, l ^ 48.
@@ -242,26 +281,25 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(SplitArgs a) {
             *reinterpret_cast<uint4*>(&qs[r][8 * ch]) = v;
         }
     }
-    // the lane's query of tile rt: row r0 + 16 rt + l16; the last position it
-    // sees (rows that are none, and tokens outside the cache, see everything
-    // and write nothing)
-    int lim[RT];
+    // the lane's query of tile rt: row r0 + 16 rt + l16, its token a whole number
+    // of tokens past tile 0's (G divides 16); rows that are none, and tokens
+    // outside the cache, see everything and write nothing
+    const int pos0 = base + ((r0 + l16) >> a.lg), tok = 16 >> a.lg;
     bool out[RT];
-    int64_t sco[RT];   // the query's row of sc, position 4 lq
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const int rr = r0 + 16 * rt + l16, pos = base + (rr >> a.lg);
-        out[rt] = rr < rows && pos >= 0 && pos < a.max_pos;
-        lim[rt] = out[rt] ? pos : 0x7FFFFFFF;
-        sco[rt] = ((int64_t)(rr >> a.lg) * a.Hq + g * G + (rr & (G - 1))) * a.max_pos + 4 * lq;
-    }
+    for (int rt = 0; rt < RT; ++rt) out[rt] = r0 + 16 * rt + l16 < rows && pos0 + rt * tok >= 0 && pos0 + rt * tok < a.max_pos;
+    // the query's row of sc, position 4 lq
+    float* const sc0 = a.sc + ((int64_t)((r0 + l16) >> a.lg) * a.Hq + g * G + (l16 & (G - 1))) * a.max_pos + 4 * lq;
+    const int64_t sc_tile = (int64_t)tok * a.Hq * a.max_pos;
     const int lim_min = base + (r0 >> a.lg);
     float m[RT], l[RT];
+    bool wide[RT];   // uniform: a row's reference is past kWide
     mx::v4f acc[RT][8];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-        m[rt] = -INFINITY;
+        m[rt] = kNone;
         l[rt] = 0.0f;
+        wide[rt] = false;
 #pragma unroll
         for (int c = 0; c < 8; ++c) acc[rt][c] = mx::v4f{0.f, 0.f, 0.f, 0.f};
     }
@@ -270,19 +308,14 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(SplitArgs a) {
         const int p0 = u * kUnit;
         const bool more = u + 4 < u1;
         uint4 kd[2][4];
-        uint32_t e15 = 0;
-        decode_k<false>(rk, kd, e15);
-        if (__ballot((e15 & 0x80808080u) != 0u)) {
-            uint32_t none = 0;
-            decode_k<true>(rk, kd, none);
-        }
+        decode_k(rk, kd);
         ko += 4 * kUnit * rs;
         if (more) load_k(rk, bk, ko, rs);
-        uint4 bh[RT], bl[RT];   // P of each row tile: high and low parts
+        uint4 p[RT][3];   // P of each row tile in three parts
         const bool masked = p0 + kUnit - 1 > lim_min;   // uniform
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            if (rt > 0 && r0 + 16 * rt >= rows) break;   // uniform: no rows left
+            if (rt > 0 && r0 + 16 * rt >= rows) break;
             mx::v4f s[2] = {mx::v4f{0.f, 0.f, 0.f, 0.f}, mx::v4f{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt) {
@@ -294,16 +327,16 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(SplitArgs a) {
             }
             // s[t][i]: position p0 + 16 t + 4 lq + i
             if (a.sc) {
-                float* row = a.sc + sco[rt] + p0;
+                float* row = sc0 + (rt * sc_tile + p0);
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    const int p = p0 + 16 * t + 4 * lq;
+                    const int pp = p0 + 16 * t + 4 * lq;
                     if (a.sc_vec && !masked) {
                         if (out[rt]) __builtin_nontemporal_store(s[t], reinterpret_cast<mx::v4f*>(row + 16 * t));
                     } else if (out[rt]) {
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            if (p + i <= lim[rt]) row[16 * t + i] = s[t][i];
+                            if (pp + i <= pos0 + rt * tok) row[16 * t + i] = s[t][i];
                     }
                 }
             }
@@ -312,21 +345,18 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(SplitArgs a) {
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        if (p0 + 16 * t + 4 * lq + i > lim[rt]) s[t][i] = -INFINITY;
+                        if (out[rt] && p0 + 16 * t + 4 * lq + i > pos0 + rt * tok) s[t][i] = -INFINITY;
             }
-            float mx_ = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                              fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-            mx_ = max_over_lq(mx_) * a.c;
             // m is the reference of the row's terms, not their maximum: it follows
             // the maximum only past a factor of 2^kSlack (any reference gives the
-            // same quotient; the sums of a first unit need no rescaling at all).
-            // It stays 2^kHead below it, so that what fp16 cuts off a term
-            // (2^-24) is 2^-31 of the largest: a row with one large score and
-            // thousands of small ones keeps the small ones' sum
-            if (__ballot(mx_ > m[rt] + (kHead + kSlack))) {
-                const float mn = fmaxf(m[rt], mx_ - kHead);
+            // same quotient; the sums of a first unit need no rescaling at all), so
+            // that the row's lanes need not agree on a maximum at every unit
+            const float top = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                                    fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+            if (__ballot(top * a.c > m[rt] + kSlack)) {
+                const float mn = fmaxf(m[rt], max_over_lq(top) * a.c);
                 if (u != u0 + wave) {
-                    const float al = __builtin_amdgcn_exp2f(m[rt] - (mn == -INFINITY ? 0.0f : mn));
+                    const float al = __builtin_amdgcn_exp2f(m[rt] - mn);
                     l[rt] *= al;
 #pragma unroll
                     for (int c = 0; c < 8; ++c)
@@ -334,42 +364,32 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(SplitArgs a) {
                         for (int i = 0; i < 4; ++i) acc[rt][c][i] *= al;
                 }
                 m[rt] = mn;
+                wide[rt] = __ballot(fabsf(mn) > kWide && mn != kNone) != 0ull;
             }
-            const float mref = m[rt] == -INFINITY ? 0.0f : m[rt];   // nothing seen yet: exp2(-inf) = 0
-            uint32_t ph[4], pl[4];
-            float sum = 0.0f;
+            float t[8];
+            if (!wide[rt]) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+                for (int i = 0; i < 8; ++i) t[i] = fmaf(s[i >> 2][i & 3], a.c, -m[rt]);
+            } else {   // the rounded product, as in m: the fma's would differ from it by more than a term
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const float a0 = __builtin_amdgcn_exp2f(fmaf(s[t][2 * i], a.c, -mref));
-                    const float a1 = __builtin_amdgcn_exp2f(fmaf(s[t][2 * i + 1], a.c, -mref));
-                    sum += a0 + a1;
-                    const f16x2_t h = __builtin_bit_cast(f16x2_t, __builtin_amdgcn_cvt_pkrtz(a0, a1));
-                    ph[2 * t + i] = __builtin_bit_cast(uint32_t, h);
-                    pl[2 * t + i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a0 - (float)h[0], a1 - (float)h[1]));
-                }
-            l[rt] += sum;
-            bh[rt] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-            bl[rt] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-        }
-        uint4 vd[8];
-        e15 = 0;
-        decode_v<false>(rv, vd, e15);
-        if (__ballot((e15 & 0x80808080u) != 0u)) {
-            uint32_t none = 0;
-            decode_v<true>(rv, vd, none);
+                for (int i = 0; i < 8; ++i) t[i] = mul_then_sub(s[i >> 2][i & 3], a.c, m[rt]);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) t[i] = __builtin_amdgcn_exp2f(t[i]);
+            l[rt] += ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+            parts(t, p[rt]);
         }
         vo += 4 * kUnit * rs;
+        uint4 vd[8];
+        decode_v(rv, vd);
         if (more) load_v(rv, bv, vo, rs);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             if (rt > 0 && r0 + 16 * rt >= rows) break;
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                acc[rt][c] = mfma_f16(vd[c], bh[rt], acc[rt][c]);
-                acc[rt][c] = mfma_f16(vd[c], bl[rt], acc[rt][c]);
-            }
+            for (int c = 0; c < 8; ++c)
+#pragma unroll
+                for (int j = 2; j >= 0; --j) acc[rt][c] = mfma_bf16(vd[c], p[rt][j], acc[rt][c]);
         }
     }
     // the four waves' sums of each tile in LDS, then one record per row: acc[rt][c][i]
@@ -393,11 +413,10 @@ __global__ __launch_bounds__(256, 2) void attn_split_kernel(SplitArgs a) {
         const int rr = r0 + 16 * rt + qr, pos = base + (rr >> a.lg);
         if (rr >= rows || pos < 0 || pos >= a.max_pos || u0 * kUnit > pos) continue;   // no record: the merge reads none
         const float gm = fmaxf(fmaxf(mm[0][qr], mm[1][qr]), fmaxf(mm[2][qr], mm[3][qr]));
-        const float gref = gm == -INFINITY ? 0.0f : gm;
         float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, den = 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-            const float wt = __builtin_amdgcn_exp2f(mm[w][qr] - gref);
+            const float wt = __builtin_amdgcn_exp2f(mm[w][qr] - gm);
             den = fmaf(wt, ml[w][qr], den);
             const float4 x = *reinterpret_cast<const float4*>(&mo[w][qr][c0]), y = *reinterpret_cast<const float4*>(&mo[w][qr][c0 + 4]);
             o[0] = fmaf(wt, x.x, o[0]); o[1] = fmaf(wt, x.y, o[1]); o[2] = fmaf(wt, x.z, o[2]); o[3] = fmaf(wt, x.w, o[3]);

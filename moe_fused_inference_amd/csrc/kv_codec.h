@@ -73,8 +73,6 @@ __device__ __forceinline__ uint32_t e4m3_encode(float v, int codec) {
 }
 
 // ---- many bytes at a time, by the hardware's OCP E4M3 conversion
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-
 // Four codec bytes as OCP E4M3 bytes of the same values; bit 7 of a byte of
 // `e15` is set when that byte's exponent field is 15 (then the result is not
 // used).
@@ -87,24 +85,16 @@ __device__ __forceinline__ uint32_t codec_to_ocp(uint32_t w, uint32_t& e15) {
     return (w & keep) | (sub & ~keep);
 }
 
-// Bytes 2 HI, 2 HI + 1 of w as two bf16 (K) or fp16 (V).  EXP15: the bytes
-// whose bit 7 is set in f had exponent 15 and are in w with exponent 14; the
-// codec reads them as 56 (8 + m), 3.5 times that (exact in both).
-template <bool HI, bool F16, bool EXP15>
+// Bytes 2 HI, 2 HI + 1 of w as two bf16.  EXP15: the bytes whose bit 7 is set in
+// f had exponent 15 and are in w with exponent 14; the codec reads them as
+// 56 (8 + m), 3.5 times that (exact).
+template <bool HI, bool EXP15>
 __device__ __forceinline__ uint32_t pair_of(uint32_t w, uint32_t f) {
-    if constexpr (F16) {
-        const f16x2_t r = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, HI);
-        if constexpr (!EXP15) return __builtin_bit_cast(uint32_t, r);
-        const f16x2_t k = {(_Float16)(f & (HI ? 0x800000u : 0x80u) ? 3.5f : 1.0f),
-                           (_Float16)(f & (HI ? 0x80000000u : 0x8000u) ? 3.5f : 1.0f)};
-        return __builtin_bit_cast(uint32_t, r * k);
-    } else {
-        const uint32_t r = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI));
-        if constexpr (!EXP15) return r;
-        const float a = __uint_as_float(r << 16) * (f & (HI ? 0x800000u : 0x80u) ? 3.5f : 1.0f);
-        const float b = __uint_as_float(r & 0xFFFF0000u) * (f & (HI ? 0x80000000u : 0x8000u) ? 3.5f : 1.0f);
-        return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xFFFF0000u);
-    }
+    const uint32_t r = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI));
+    if constexpr (!EXP15) return r;
+    const float a = __uint_as_float(r << 16) * (f & (HI ? 0x800000u : 0x80u) ? 3.5f : 1.0f);
+    const float b = __uint_as_float(r & 0xFFFF0000u) * (f & (HI ? 0x80000000u : 0x8000u) ? 3.5f : 1.0f);
+    return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xFFFF0000u);
 }
 
 // A codec word ready for pair_of, and its exponent-15 flags.

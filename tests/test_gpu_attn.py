@@ -219,26 +219,53 @@ def test_attn_decode_split_vs_oracle(dext, M, Hq, Hkv, max_pos, base):
     assert torch.isnan(sc[live[0], :, base + live[0] + 1:]).all()
 
 
-def test_attn_decode_split_one_large_score(dext):
+# one score of q * sqrt(128) / 16 of a context's n = base + 1 .. positions, 0 for the others; the values' codes at that
+# position and at the others.  The weight of a small score against the large one is rounded in its exponent (below 2^5, so
+# by 2^-20) where the scores' scale is applied, where a wave takes its reference and where records are merged: 3 * 2^-20 *
+# ln 2 = 2e-6, which the result follows where the small terms make it up, and by a fortieth of that in the first case
+@pytest.mark.parametrize("M,Hkv,max_pos,base,a,first,rest,tol", [
+    (16, 2, 65536, 65515, 1.546875, 0x38, 0x58, 1e-6),     # e^17.5 against 65520 ones, values 1 and 16
+    (16, 2, 65536, 65515, 1.546875, 0x01, 0x78, 3e-6),     # values 2^-6 and 448
+    (16, 2, 65536, 65515, 1.890625, 0x01, 0x78, 3e-6),     # e^21.4
+    (9, 4, 23040, 22992, 1.234375, 0x01, 0x78, 3e-6),      # e^14
+    (9, 4, 23040, 22992, 1.890625, 0x00, 0x38, 3e-6),      # the large one's value is 0
+    (2, 4, 8192, 37, 1.546875, 0x01, 0x78, 3e-6),          # all in two units of one wave each
+    (5, 8, 4200, 4100, 6.0, 0x00, 0x38, 1.2e-5)])          # e^67.9: exponents up to 2^7, rounded by 2^-18
+def test_attn_decode_split_one_large_score(dext, M, Hkv, max_pos, base, a, first, rest, tol):
     """A position that takes most of the weight leaves the sum of the many small
-    ones: scores of s at position 0 and 0 elsewhere, values 1 and 16."""
-    M, Hq, Hkv, max_pos, base = 16, 32, 2, 65536, 65515
+    ones, whose probabilities keep their bits at any size."""
+    Hq = 32
     kvk = torch.zeros((max_pos, Hkv * 128), dtype=torch.uint8, device=DEV)
-    kvv = torch.full_like(kvk, 0x58)                                     # 16
-    kvk[0], kvv[0] = 0x38, 0x38                                          # 1
-    q = torch.full((M, Hq, 128), 1.546875, dtype=torch.bfloat16, device=DEV)
+    kvv = torch.full_like(kvk, rest)
+    kvk[0], kvv[0] = 0x38, first                                         # 1
+    q = torch.full((M, Hq, 128), a, dtype=torch.bfloat16, device=DEV)
     o = dext.attn_decode(q, kvk.view(max_pos, Hkv, 128), kvv.view(max_pos, Hkv, 128),
                          torch.tensor([base], dtype=torch.int32, device=DEV),
                          torch.empty((M, Hq, max_pos), dtype=torch.float32, device=DEV), M)
     torch.cuda.synchronize()
-    w = np.exp(-1.546875 * 128 / np.sqrt(128.0))                         # 2^-25.2
+    vf, vr = (float(attn.e4m3_ref_decode(np.uint8(c))) for c in (first, rest))
+    w = np.exp(-a * 128 / np.sqrt(128.0))
     n = base + np.arange(M, dtype=np.float64)
-    ref = ((1 + 16 * w * n) / (1 + w * n))[:, None, None]
-    # 2^-31 of the largest term lost on each of the 416 positions it shares a
-    # wave with, times 16: 3e-6; the wave's 26 matrix instructions add to a sum
-    # of that term's size, up to 8 times each with 2^-23 cut off: 2.5e-5 (a
-    # reference at the row's maximum would lose 16 * 416 * 2^-25.2 = 1.7e-4)
-    assert np.abs(np_(o) / ref - 1).max() <= 3e-5
+    ref = ((vf + vr * w * n) / (1 + w * n))[:, None, None]
+    err = np.abs(np_(o) / ref - 1).max()
+    log(f"  one large score, M={M} base={base} a={a}: {err:.2e}")
+    assert err <= tol
+
+
+@pytest.mark.parametrize("M,Hq,Hkv,scale", [(2, 8, 2, 28), (9, 32, 4, 28), (3, 32, 4, 60)])
+def test_attn_decode_split_scores_past_fp32_resolution(dext, M, Hq, Hkv, scale):
+    """Scores so large that their exponents are whole numbers of bits apart: the
+    largest takes all, as in the oracle."""
+    rng = np.random.default_rng(77)
+    max_pos, base = 4352, 4300
+    kvk_np, kvv_np = _cache(rng, max_pos, Hkv, 128), _cache(rng, max_pos, Hkv, 128)
+    q = _bf16(rng.standard_normal((M, Hq, 128)) * 2.0 ** scale)
+    o = dext.attn_decode(q.to(DEV), torch.from_numpy(kvk_np).to(DEV), torch.from_numpy(kvv_np).to(DEV),
+                         torch.tensor([base], dtype=torch.int32, device=DEV),
+                         torch.empty((M, Hq, max_pos), dtype=torch.float32, device=DEV), M)
+    torch.cuda.synchronize()
+    ref, _ = attn.attn_decode_ref(q.float().numpy(), kvk_np, kvv_np, base)
+    assert_close(np_(o), ref, what=f"attn split, scores of 2^{scale}, M={M}", rel_max=1e-5)
 
 
 @pytest.mark.parametrize("codec", [0, 1])
