@@ -49,6 +49,8 @@
 #include "mx_device.h"
 #include "mx_host.h"
 
+#include <algorithm>
+
 namespace {
 
 template <int BM, int BN, int BK, int NW, bool RG>
@@ -414,6 +416,20 @@ void xcd_blocks(G2Args& g) {
     g.per_xcd = ((nblk + 7) / 8) * bm * bn;
 }
 
+// The most tiles of BM x BN that an XCD gets that way.
+int64_t most_on_xcd(int M, int N, int BM, int BN) {
+    G2Args g{};
+    g.tiles_m = (M + BM - 1) / BM;
+    g.tiles_n = (N + BN - 1) / BN;
+    xcd_blocks(g);
+    int64_t n[8] = {};
+    const int xblk_m = (g.tiles_m + g.bm - 1) / g.bm;   // few: a block is about an eighth of the grid, or a row of it
+    for (int i = 0, b = 0; i < xblk_m; ++i)
+        for (int j = 0; j < g.xblk_n; ++j, ++b)
+            n[b % 8] += (int64_t)std::min(g.bm, g.tiles_m - i * g.bm) * std::min(g.bn, g.tiles_n - j * g.bn);
+    return *std::max_element(n, n + 8);
+}
+
 }  // namespace
 
 namespace mxh {
@@ -436,20 +452,36 @@ int launch_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const
 template <bool RG>
 int pick_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y, int M, int N,
                int Kp, hipStream_t st) {
-    // The tile by the number of tiles a grid gives (MI355X, us):
+    // The tile by the number of tiles a grid gives, over its CUs and over the 32
+    // CUs of the XCD that gets most (MI355X, us, a call in a graph; 355 shapes of
+    // whole K steps, M 17-6000, N 128-20000, K 256-16384, each with every instance):
     //  * at most 256 of 64 x 64 (one a CU): 64 x 64, four stages.  512 x 2048 x
     //    2048 5.9, 32 x 2048 x 4096 7.3; 64 x 128 7.6 and 9.8; eight stages
     //    (one workgroup per CU, whatever the grid) 6.9 and 8.3.
     //  * K of 1536 on and at least 160 of 256 x 256, unless half of each would be
     //    padding (t128 = 2 t256): 4096^2 x 2048 28.8 against 31.2 with 128 x 128,
-    //    2048 x 5120 x 2048 21.6 against 23.7; but 144 tiles 30.9 against 29.7,
-    //    128 tiles 20.0 against 17.5, and with less K to each output's store
-    //    4096^2 x 768 20.0 against 18.4.
-    //  * at least 160 of 128 x 128 and M > 64: 128 x 128.  1500 x 3000 x 1024
-    //    10.8 against 12.8 with 64 x 128 (15.5 with four waves and four stages, one
-    //    workgroup per CU); at 512 x 5120 x 2048, 160 tiles, 9.9 against 11.4.
-    //    With K < 1024 the smaller tile goes on a little longer: 2048 x 3000 x 768
-    //    10.7 against 11.5, 4096^2 x 768 21.0 against 18.4.
+    //    2048 x 5120 x 2048 21.6 against 23.7; with less K to each output's store
+    //    4096^2 x 768 20.0 against 18.4.  From 128 of them on where 128 x 128 takes
+    //    more than a round of two a CU and its second one is mostly idle: without
+    //    padding from K = 3072 on, 3000^2 x 3072 35.4 against 37.0 and x 8192 65.3
+    //    against 84.7, but x 2048 30.1 against 29.5 and 2560 x 3300 x 2560 33.1
+    //    against 29.9; in any case from K = 5120 on, 2100 x 3900 x 8192 64.5
+    //    against 74.5, x 4096 41.1 against 39.9.
+    //  * one 128 x 128 a CU, and more than one 64 x 128 on some: with a long K the
+    //    deeper ring (four stages, no second workgroup to hide the copies under):
+    //    512 x 6144 x 4096 13.8 against 15.1 with two stages, x 8192 25.7 against
+    //    33.0, but x 1536 8.1 against 7.6 and 900 x 3700 x 2560 12.3 against 11.8.
+    //    With a tile on nearly every CU from K = 2048 on (10.2 against 10.6), and
+    //    if they are full with four waves of 64 x 64 each: 512 x 8192 x 4096 15.9,
+    //    eight waves 16.9, two stages 16.9 (with ragged edges, 4076 x 988 x 2048:
+    //    13.9, 11.4, 11.8).
+    //  * at least 160 of 128 x 128 and M > 64: 128 x 128, two stages.  1500 x 3000
+    //    x 1024 10.8 against 12.8 with 64 x 128 (15.5 with four waves and four
+    //    stages, one workgroup per CU); at 512 x 5120 x 2048, 160 tiles, 9.9
+    //    against 11.4.  With K < 1024 the smaller tile goes on a little longer:
+    //    2048 x 3000 x 768 10.7 against 11.5, 4096^2 x 768 21.0 against 18.4.  With
+    //    fewer, where 64 x 128 would put two on a CU: 600 x 2560 x 2048 9.1 against
+    //    10.8, 1500 x 1300 x 1024 8.7 against 10.3.
     //  * else 64 x 128, three stages (two with ragged scales, to stay at two
     //    workgroups per CU): 1000 x 2000 x 2048 7.8 against 8.6 with 64 x 64, 32 x
     //    151936 x 2048 40.2 against 45.2 and 62 with 256 x 256.
@@ -461,6 +493,21 @@ int pick_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const u
     if (t64 <= 256) return launch_gemm2<64, 64, 256, 4, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
     if (Kp >= 1536 && t256 >= 160 && 2 * t128 >= 5 * t256)
         return launch_gemm2<256, 256, 256, 2, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+    if constexpr (!RG) {
+        const int cus = 32;   // of an XCD
+        const int64_t x128 = most_on_xcd(M, N, 128, 128);
+        if (t256 >= 128 && x128 > 2 * cus &&
+            ((2 * t128 >= 5 * t256 && Kp >= 5120) || (t128 == 4 * t256 && Kp >= 3072)))
+            return launch_gemm2<256, 256, 256, 2, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+        if (M > 64 && x128 <= cus && most_on_xcd(M, N, 64, 128) > cus) {
+            if (Kp >= 2048 && t128 > 240 && M % 128 == 0 && N % 128 == 0)
+                return launch_gemm2<128, 128, 256, 4, 4, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+            if (Kp >= (t128 > 240 ? 2048 : 3072))
+                return launch_gemm2<128, 128, 256, 4, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+            if (t128 < 160 && (Kp >= 768 || t64x128 > 256))
+                return launch_gemm2<128, 128, 256, 2, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
+        }
+    }
     if (M > 64 && t128 >= 160 && !(Kp < 1024 && t64x128 <= 768))
         return launch_gemm2<128, 128, 256, 2, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);
     return launch_gemm2<64, 128, 256, RG ? 2 : 3, 8, RG>(xq, xsc, wp, wsc, y, M, N, Kp, st);

@@ -66,7 +66,10 @@ RAGGED_SHAPES = [(17, 33, 32), (65, 127, 224), (333, 1000, 2080), (100, 129, 131
 # the tile rule's other sides: M up to one and just past one 64- and 128-row tile with many columns, 144 and 160 tiles of
 # 256 x 256, K on both sides of 1024 and 1536
 @pytest.mark.parametrize("M,N,K", [(64, 5000, 512), (65, 10300, 512), (129, 5300, 1024), (2300, 4000, 1536), (2500, 4090, 1536),
-                                   (2300, 2500, 1280), (520, 5121, 2048)])
+                                   (2300, 2500, 1280), (520, 5121, 2048),
+                                   # a long K with one 128 x 128 a CU: full tiles, ragged ones, one XCD short of them; 135 tiles of
+                                   # 256 x 256 without padding; two stages of 128 x 128 below 160 tiles
+                                   (1024, 4096, 2048), (1000, 4001, 2304), (500, 5900, 3072), (2304, 3840, 3072), (1500, 1300, 512)])
 def test_lin_pq_tile_rule_vs_oracle(dext, M, N, K):
     test_lin_pq_vs_oracle(dext, M, N, K)
 
