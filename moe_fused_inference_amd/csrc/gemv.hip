@@ -899,16 +899,27 @@ int lin_pq_gemv(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const 
     return MXFP4_OK;
 }
 
-// Stages (row tiles x K / 1024) from which the streaming kernel takes over,
-// four per wave: with fewer its start, the first copies' latency and the
-// activation rows, shows (MI355X, us, tile per wave / streaming: 2048 stages
-// 16384 x 2048 7.3 / 7.3 and 32768 x 1024 6.1 / 7.0, 3000 stages 24000 x 2048
-// 10.4 / 9.3, 4096 stages 16384 x 4096 13.3 / 11.2 and 32768 x 2048 11.3 /
-// 10.8, 18992 stages 151936 x 2048 42.5 / 34.5).  With one stage a tile the
-// ring is drained by half as much work per output, so it takes more of them:
-// 65536 x 1024 is 11.1 / 10.6 with eight rows but 9.4 / 10.1 with one, 98400 x
-// 1024 15.3 / 13.6 and 12.7 / 13.0, 151936 x 1024 17.7 / 17.6 with one.
-constexpr int kStreamStages = 4096, kStreamStages1 = 8192;
+// Stages (row tiles x K / 1024) from which the streaming kernel takes over (a
+// wave has four at 4096): with fewer its start, the first copies' latency and
+// the activation rows, shows.  MI355X, us, tile per wave / streaming, weights in
+// the Infinity Cache (from HBM the streaming kernel is ahead by 5 to 10 % more):
+//   2048 x 32768, 4096 stages   M = 1 10.5 / 11.3  M = 4 11.2 / 11.3  M = 16 13.4 / 12.1
+//   2048 x 40000, 5000          M = 1 14.0 / 13.2  M = 4 15.1 / 13.3  M = 16 18.7 / 13.9
+//   3072 x 21846, 4098          M = 1 12.4 / 11.1  M = 4 13.7 / 11.5  M = 16 17.2 / 12.6
+//   4096 x 16384, 4096          M = 1 12.7 / 11.2  M = 4 13.5 / 11.7  M = 16 15.5 / 13.1
+//   2048 x 151936, 18992        M = 1 37.1 / 32.9  M = 4 40.4 / 33.4  M = 16 51.2 / 36.8
+// so at K = 2048 one and two rows take it past 4096 only.  (Below, sizes that
+// leave the tile-per-wave kernel a nearly empty last round would gain too, 24000 x
+// 2048 10.4 / 9.3 with eight rows, and those that do not lose, 16384 x 2048 7.3 /
+// 7.3 and 32768 x 1024 6.1 / 7.0.)  With one stage a tile the ring is drained by
+// half as much work per output, so it takes more of them: 65536 x 1024 is 11.1 /
+// 10.6 with eight rows but 9.4 / 10.1 with one, 131072 x 1024 20.8 / 19.0 and 17.8
+// / 18.0, 151936 x 1024 23.6 / 20.3 and 20.3 / 19.6.
+bool lin_streams(int M, int Kp, int tiles) {
+    const int stages = tiles * (Kp / kStK);
+    if (Kp == kStK) return stages >= 8192;
+    return Kp == 2 * kStK && M <= 2 ? stages > 4096 : stages >= 4096;
+}
 
 template <int NST>
 int launch_lin_stream_n(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const uint8_t* wsc, float* y, int M,
@@ -938,7 +949,7 @@ int lin_small(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const ui
               int Kp, hipStream_t st) {
     const int tiles = (N + 15) / 16;
     const int steps = (Kp / 32 + 3) / 4;
-    if (Kp % kStK == 0 && Kp <= 4096 && N <= (1 << 24) && tiles * (Kp / kStK) >= (Kp > kStK ? kStreamStages : kStreamStages1) &&
+    if (Kp % kStK == 0 && Kp <= 4096 && N <= (1 << 24) && lin_streams(M, Kp, tiles) &&
         ((((uintptr_t)xq | (uintptr_t)xsc | (uintptr_t)wp | (uintptr_t)wsc) & 15) == 0))
         return launch_lin_stream(xq, xsc, wp, wsc, y, M, N, Kp, tiles, st);
     int S = 1;
