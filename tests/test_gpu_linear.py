@@ -80,26 +80,29 @@ def test_lin_pq_ragged_k_vs_oracle(dext, M, N, K):
 
 
 # the streaming GEMV of a many-row weight: its smallest sizes at each K, a last tile of one row, waves with a tile fewer,
-# one to sixteen activation rows
-@pytest.mark.parametrize("M,N,K", [(1, 32768, 2048), (8, 131089, 1024), (16, 22001, 3072), (5, 16400, 4096)])
-def test_lin_pq_streamed_rows(dext, M, N, K):
+# one to sixteen activation rows; `part`: rows of a slice that is too short to stream and long enough to leave K whole
+# (1024 tiles and more; at K = 4096 so many stream)
+@pytest.mark.parametrize("M,N,K,part", [(1, 32784, 2048, 16384), (3, 32768, 2048, 16384), (8, 131089, 1024, 65536),
+                                        (16, 22001, 3072, 16384), (5, 16400, 4096, None), (1, 40001, 4096, None)])
+def test_lin_pq_streamed_rows(dext, M, N, K, part):
     """Equal, bit for bit, to the same rows as slices of fewer rows, which
     take the kernel of a tile per wave (its unsplit instance: the same MFMA
-    chain)."""
+    chain); the last slice ends at N.  Where there is none, every row against
+    the oracle."""
     g = torch.Generator(device=DEV)
     g.manual_seed(M + N)
     wp, wsc = dext.prequant(torch.randn((N, K), generator=g, device=DEV).bfloat16())
     xq, xs = dext.prequant(torch.randn((M, K), generator=g, device=DEV).bfloat16())
     y = dext.lin_pq(xq, xs, wp, wsc, M, N, K)
-    for n0 in range(0, N, 16384):
-        n1 = min(N, n0 + 16384)
-        if n1 - n0 < 16384 or (n1 - n0) // 16 * (K // 1024) >= (4096 if K > 1024 else 8192):
-            continue
-        assert torch.equal(dext.lin_pq(xq, xs, wp[n0:n1].contiguous(), wsc[n0:n1].contiguous(), M, n1 - n0, K),
-                           y[:, n0:n1])
-    # the whole of it against fp32 products of the same operands, summed in fp64
-    rows = torch.cat((torch.arange(0, min(N, 300)), torch.arange(N - 300, N))).to(DEV)
-    want = ops.lin_pq_ref(np_(xq), np_(xs), np_(wp[rows]), np_(wsc[rows]))
+    if part:
+        for n0 in [*range(0, N - part, part), N - part]:   # (N - part: any row may be a slice's first)
+            n1 = n0 + part
+            assert torch.equal(dext.lin_pq(xq, xs, wp[n0:n1].contiguous(), wsc[n0:n1].contiguous(), M, part, K), y[:, n0:n1])
+        rows = torch.cat((torch.arange(0, 300), torch.arange(N - 300, N))).to(DEV)
+    else:
+        rows = torch.arange(N, device=DEV)
+    # against fp32 products of the same operands, summed in fp64
+    want = ops.lin_pq_ref_chunked(np_(xq), np_(xs), np_(wp[rows]), np_(wsc[rows]))
     assert_close(np_(y[:, rows]), want, what=f"lin_pq streamed {M}x{N}x{K}")
 
 
