@@ -309,11 +309,8 @@ __global__ __launch_bounds__(256) void argmax_kernel(const float* __restrict__ l
     }
 }
 
-size_t argmax_ws_bytes(int M, int V) {
-    const int64_t P = (V + kArgSlice - 1) / kArgSlice;
-    const int64_t head = ((int64_t)(M + 1) * 4 + 255) / 256 * 256;
-    return (size_t)(head + 2 * (int64_t)M * P * 4);
-}
+size_t argmax_ws_head(int M) { return ((size_t)(M + 1) * 4 + 255) / 256 * 256; }   // the counters
+size_t argmax_ws_bytes(int M) { return argmax_ws_head(M) + (size_t)M * 8; }
 
 }  // namespace
 
@@ -363,20 +360,19 @@ extern "C" int mxfp4_qk_norm_rope_kv(const float* qkv, const void* q_norm_w, con
 
 extern "C" size_t mxfp4_argmax_workspace_size(int M, int V) {
     if (M <= 0 || V <= 0) return 0;
-    return argmax_ws_bytes(M, V);
+    return argmax_ws_bytes(M);
 }
 
 extern "C" int mxfp4_argmax_advance(const float* logits, int M, int V, int32_t* ids, int32_t* dpos, void* ws,
                                     size_t ws_bytes, void* stream) {
     MXH_REQUIRE(logits && ids && ws, "argmax_advance: null pointer");
     MXH_REQUIRE(M > 0 && M <= 65535 && V > 0, "argmax_advance: M=%d V=%d", M, V);
-    MXH_REQUIRE(ws_bytes >= argmax_ws_bytes(M, V), "argmax_advance: workspace of %zu bytes, %zu needed", ws_bytes,
-                argmax_ws_bytes(M, V));
+    MXH_REQUIRE(ws_bytes >= argmax_ws_bytes(M), "argmax_advance: workspace of %zu bytes, %zu needed", ws_bytes,
+                argmax_ws_bytes(M));
     MXH_REQUIRE(((uintptr_t)ws & 255) == 0, "argmax_advance: workspace must be 256-byte aligned");
     const int P = (V + kArgSlice - 1) / kArgSlice;
-    const int64_t head = ((int64_t)(M + 1) * 4 + 255) / 256 * 256;
     uint8_t* w = static_cast<uint8_t*>(ws);
-    ArgWs a{reinterpret_cast<uint32_t*>(w), reinterpret_cast<uint64_t*>(w + head)};
+    ArgWs a{reinterpret_cast<uint32_t*>(w), reinterpret_cast<uint64_t*>(w + argmax_ws_head(M))};
     hipLaunchKernelGGL(argmax_kernel, dim3(P, M), dim3(256), 0, mxh::as_stream(stream), logits, V, M, ids, dpos, a);
     return mxh::launch_status("argmax_advance");
 }

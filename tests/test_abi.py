@@ -47,8 +47,9 @@ def test_workspace_size(lib):
     # and H x words, per slot H y words
     assert lib.mxfp4_decode_stack_workspace_size(8, 2048, 768) == 2048 + 2 * 8 * (2 * 768 + 2048 + 2048) * 8
     assert lib.mxfp4_decode_stack_workspace_size(0, 2048, 768) == 0
-    # argmax: 256-byte counter head, then (M, P) maxima and indices, P = ceil(V / 4096) slices
-    assert lib.mxfp4_argmax_workspace_size(8, 151936) == 256 + 2 * 8 * 38 * 4
+    # argmax: 256-byte counter head, then a 64-bit key per row
+    assert lib.mxfp4_argmax_workspace_size(8, 151936) == 256 + 8 * 8
+    assert lib.mxfp4_argmax_workspace_size(64, 100) == 512 + 64 * 8
     assert lib.mxfp4_argmax_workspace_size(0, 100) == 0
 
 

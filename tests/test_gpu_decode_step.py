@@ -319,6 +319,30 @@ def test_argmax_slices_match_torch(V):
     assert int(ws[:head].count_nonzero()) == 0, "row counters not reset"
 
 
+@pytest.mark.parametrize("M,V", [(1, 151936), (5, 12289), (70, 4097), (3, 100)])
+def test_argmax_leaves_nothing_behind(M, V):
+    """Calls on one workspace whose maxima fall from call to call (a key left
+    behind would win), rows without a number after rows with one, all -inf,
+    signed zeros; other shapes in between; every byte is zero after each."""
+    lib = _lib.load()
+    g = torch.Generator(device=DEV)
+    g.manual_seed(M + V)
+    ws = torch.zeros(lib.mxfp4_argmax_workspace_size(M, V), dtype=torch.uint8, device=DEV)
+    ids = torch.empty(M, dtype=torch.int32, device=DEV)
+    lg = torch.randn((M, V), generator=g, device=DEV)
+    falling = [lg + 100.0, lg, lg - 1e6, torch.full_like(lg, float("nan")), torch.full_like(lg, -float("inf")),
+               -torch.zeros_like(lg), -lg.abs() - 1e30]
+    falling[3][-1, V // 2] = -3e38                      # one finite value among NaNs in the last row
+    falling[5][:, V - 1] = 0.0                          # 0 equals -0: the first index
+    for call, x in enumerate(falling):
+        _argmax(lib, x.contiguous(), ids, None, ws)
+        want = sref.argmax_ref(np.where(np.isnan(np_(x)), -np.inf, np_(x)))
+        assert np.array_equal(np_(ids), want), call
+        assert int(ws.count_nonzero()) == 0, f"call {call}"
+        _argmax(lib, lg[:1, :1 + V // 2].contiguous(), ids[:1], None, ws)
+        assert int(ws.count_nonzero()) == 0, f"one row after call {call}"
+
+
 @pytest.mark.parametrize("M,Hq,Hkv,max_pos,base,codec", [
     (1, 32, 4, 4096, 4093, 0),    # the config-5 step: the new row in the last chunk
     (1, 32, 4, 4096, 64, 0),      # the new row first in its chunk
