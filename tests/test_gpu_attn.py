@@ -219,6 +219,33 @@ def test_attn_decode_split_vs_oracle(dext, M, Hq, Hkv, max_pos, base):
     assert torch.isnan(sc[live[0], :, base + live[0] + 1:]).all()
 
 
+# fewer splits than 128-position pieces of the cache, so a split's share follows the context (attn_split.hip's
+# units_per_split): 128, 64, 42 and 32 splits (each merge kernel), one, two and three row tiles; a cache that is full, one
+# that is nearly empty (the share at its floor), tokens on both sides of a split's edge, the first of a new round of shares;
+# q of standard deviation 1, and 4, whose softmax spreads over more than 2^20
+@pytest.mark.parametrize("M,Hq,Hkv,max_pos,base,qs", [
+    (4, 32, 4, 23040, 23036, 1), (4, 32, 4, 23040, 700, 1), (4, 32, 4, 23040, 19966, 4), (4, 32, 4, 23040, 16380, 1),
+    (9, 32, 4, 16640, 16631, 1), (9, 32, 4, 16640, 250, 4), (9, 32, 4, 16640, 12283, 4), (16, 32, 4, 8448, 8432, 1),
+    (16, 32, 4, 8448, 5368, 1), (16, 32, 8, 8448, 8000, 4), (2, 8, 8, 16640, 16500, 1), (2, 8, 8, 16640, 8191, 4)])
+def test_attn_decode_split_shares_vs_oracle(dext, M, Hq, Hkv, max_pos, base, qs):
+    """As test_attn_decode_split_vs_oracle where splits are shares of the context."""
+    rng = np.random.default_rng(M * 13 + max_pos + base)
+    kvk_np, kvv_np = _cache(rng, max_pos, Hkv, 128), _cache(rng, max_pos, Hkv, 128)
+    kvv_np[3::97] = _cache(rng, max_pos, Hkv, 128, 300.0)[3::97]
+    q = _bf16(rng.standard_normal((M, Hq, 128)) * qs)
+    sc = torch.full((M, Hq, max_pos), float("nan"), dtype=torch.float32, device=DEV)
+    o = dext.attn_decode(q.to(DEV), torch.from_numpy(kvk_np).to(DEV), torch.from_numpy(kvv_np).to(DEV),
+                         torch.tensor([base], dtype=torch.int32, device=DEV), sc, M)
+    torch.cuda.synchronize()
+    ref, scores = attn.attn_decode_ref(q.float().numpy(), kvk_np, kvv_np, base)
+    assert_close(np_(o), ref, what=f"attn shares M={M} Hq={Hq} Hkv={Hkv} base={base} q*{qs}", rel_max=1e-5)
+    for m in range(M):
+        S = base + m + 1
+        err = np.abs(np_(sc[m, :, :S]).astype(np.float64) - scores[m]).max() / np.abs(scores[m]).max()
+        assert err <= 1e-5, (m, err)
+        assert torch.isnan(sc[m, :, S:]).all()
+
+
 # one score of q * sqrt(128) / 16 of a context's n = base + 1 .. positions, 0 for the others; the values' codes at that
 # position and at the others.  The weight of a small score against the large one is rounded in its exponent (below 2^5, so
 # by 2^-20) where the scores' scale is applied, where a wave takes its reference and where records are merged: 3 * 2^-20 *
