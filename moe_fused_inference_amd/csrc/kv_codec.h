@@ -9,16 +9,6 @@
 
 namespace kv {
 
-// The reference's E4M3 byte -> float.
-__device__ __forceinline__ float e4m3_ref_decode(uint32_t b) {
-    const uint32_t e = (b >> 3) & 15u, m = b & 7u;
-    float v;
-    if (e == 0) v = (float)m * 0.015625f;                       // m * 2^-6
-    else if (e == 15) v = (float)(8u + m) * 56.0f;              // 448 * (1 + m/8)
-    else v = __uint_as_float(((e + 120u) << 23) | (m << 20));   // (1 + m/8) * 2^(e-7)
-    return (b & 0x80u) ? -v : v;
-}
-
 // The reference's float -> E4M3 byte (round half away from zero).
 __device__ __forceinline__ uint32_t e4m3_ref_encode(float v) {
     const uint32_t sign = v < 0.0f ? 0x80u : 0u;

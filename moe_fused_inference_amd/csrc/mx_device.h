@@ -180,12 +180,6 @@ __device__ __forceinline__ v4f mfma16_fp8a_fp4b(v8i a, uint4 b, v4f c, uint32_t 
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, bv, c, 0, 4, 0, (int)sa, 0, (int)sb);
 }
 
-__device__ __forceinline__ v16f mfma32_fp4(uint4 a, uint4 b, v16f c, uint32_t sa, uint32_t sb) {
-    v8i av = {(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
-    v8i bv = {(int)b.x, (int)b.y, (int)b.z, (int)b.w, 0, 0, 0, 0};
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, c, 4, 4, 0, (int)sa, 0, (int)sb);
-}
-
 // Materialises an MFMA result at this point of wave-uniform control flow.
 // An MFMA reads the operands of all 64 lanes, but the compiler models it as a
 // per-lane operation: when only some lanes consume the result (`if (lane <
