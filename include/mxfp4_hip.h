@@ -152,6 +152,11 @@ int mxfp4_moe_combine(const float* yd, int ystride, const float* w, int E,
  *   workspace  16-byte aligned device memory of
  *              mxfp4_attn_decode_workspace_size(M, Hq, max_pos) bytes (the
  *              softmax partials; nothing persists)
+ * Up to max_pos 4096 a token's result is the same, bit for bit, whatever M it
+ * comes with.  Past it the softmax of one token is summed over 64-position
+ * chunks and that of several over shares of the context that depend on M and
+ * *dpos, so the same token may differ between such calls by the rounding of
+ * its sums (relative 2e-6).
  */
 size_t mxfp4_attn_decode_workspace_size(int M, int Hq, int max_pos);
 int mxfp4_attn_decode(const void* q, const uint8_t* kvk, const uint8_t* kvv, const int32_t* dpos,
@@ -187,8 +192,9 @@ int mxfp4_attn_decode_fused(const float* qkv, const void* q_norm_w, const void* 
                             uint8_t* oq, uint8_t* os, int M, int Hq, int Hkv, int D, int max_pos, int codec,
                             void* workspace, size_t workspace_bytes, void* stream);
 
-/* mxfp4_attn_decode_fused_partials: the first pass of mxfp4_attn_decode_fused
- * alone -- q/k norm, RoPE, the KV write and every 64-position chunk's softmax
+/* mxfp4_attn_decode_fused_partials: the chunk pass of mxfp4_attn_decode_fused
+ * alone (its first pass for M = 1 and for max_pos <= 4096; this entry takes it
+ * for any) -- q/k norm, RoPE, the KV write and every 64-position chunk's softmax
  * record -- leaving the records in the workspace for the merge that
  * mxfp4_decode_layer_post_attn runs at the front of the MoE launch (no merge
  * launch here).  Arguments as mxfp4_attn_decode_fused without outputs. */

@@ -123,15 +123,26 @@ int launch_attn(const void* q, const uint8_t* kvk, const uint8_t* kvv, const int
                 "attn_decode: workspace must be 16-byte aligned and hold mxfp4_attn_decode_workspace_size bytes");
     const int G = Hq / Hkv;
     // Several tokens over a cache of more than 64 chunks: the context-split
-    // kernel (attn_split.hip) for every entry, so that they go on agreeing bit
-    // for bit.  The chunk pass writes a record per token, head and 64 positions
-    // there (55 MB at 9 tokens and 23001 positions, more than the cache's 24)
-    // and decodes each byte for 4 tokens at a time.  One token stays on chunks,
-    // whose records the layer launch merges, and so does a short cache, where
-    // both wait on latency: 4096 positions, 1 token 9.8 against 8.4 us, 9 tokens
-    // 19.6 against 15.4; 23001 positions, 4 tokens 29.5 against 19.2, 9 tokens
-    // 54.4 against 25.2, 16 tokens 73.6 against 34.0.  (It addresses a cache
-    // with 31-bit offsets.)
+    // kernel (attn_split.hip), in attn_decode, _mx and _fused alike, so that
+    // these go on agreeing bit for bit.  The chunk pass writes a record per
+    // token, head and 64 positions there (55 MB at 9 tokens and 23001 positions,
+    // more than the cache's 24) and decodes each byte for 4 tokens at a time.
+    // MI355X, us a call, chunks / split, 32 / 4 heads, no raw scores kept:
+    //   max_pos, context   M = 2         M = 4         M = 9         M = 16
+    //    8192,  8000       15.4 / 10.1   18.9 / 13.1   27.4 / 18.8   31.3 / 22.7
+    //   23296, 23001       22.5 / 17.0   27.3 / 20.7   48.8 / 25.1   65.8 / 33.1
+    //   32768,   500       10.9 /  9.7   13.9 / 12.3   16.9 / 14.7   17.9 / 14.8
+    //   the last, _fused   13.3 / 12.6   17.0 / 15.3   20.7 / 18.1   24.2 / 18.1
+    //    4096,  4000       10.3 /  8.6   12.9 / 11.1   17.6 / 14.3   21.7 / 17.0
+    //    4096,   500        8.5 /  8.3   10.1 / 10.5   13.0 / 12.8   15.5 / 14.0
+    // It would serve most of 4096 and below as well; the line is where the
+    // workspace, whose size callers know, has room for _fused's q past the
+    // records.  One token stays on chunks at any length, though longer ones would
+    // gain too (8000 positions 14.3 / 10.3, 23001 21.2 / 17.4): its records are
+    // what the layer launch writes and merges.  So past 4096 positions a token's
+    // bits depend on M, on the path for one or several and through the number of
+    // splits and their bounds; up to there they do not.  (The split kernel
+    // addresses a cache with 31-bit offsets.)
     if (M > 1 && max_pos > 64 * kChunk && merge && G <= 16 && (G & (G - 1)) == 0 &&
         (int64_t)max_pos * Hkv * kD < (1ll << 31)) {
         if constexpr (FUSED) {

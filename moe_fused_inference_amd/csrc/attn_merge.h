@@ -34,7 +34,7 @@ struct MergeLds {
 // loads in flight.  The four phases meet in LDS.  Returns true in wave 0,
 // whose lane l then holds o[2l], o[2l+1] in r0, r1; the other waves return
 // false and must not wait at a barrier afterwards.  LOG2: the records'
-// maxima are in base 2 (the sums of exp2(s - m_c)).
+// m_c are references in base 2 (the sums of exp2(s - m_c)), not maxima.
 template <bool LOG2 = false>
 __device__ __forceinline__ bool merge_head(const float* rec, int n, MergeLds& s, float& r0, float& r1) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

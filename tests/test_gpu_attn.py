@@ -295,6 +295,31 @@ def test_attn_decode_split_scores_past_fp32_resolution(dext, M, Hq, Hkv, scale):
     assert_close(np_(o), ref, what=f"attn split, scores of 2^{scale}, M={M}", rel_max=1e-5)
 
 
+@pytest.mark.parametrize("Hq,Hkv,max_pos,base", [(32, 4, 4096, 4000), (8, 8, 4096, 63), (32, 4, 4352, 4200)])
+def test_attn_decode_token_alone_and_in_company(dext, Hq, Hkv, max_pos, base):
+    """A token's result up to max_pos 4096 has the same bits in any company;
+    past it, one token and several take different sums of the same terms: the
+    chunk pass's 16 bits of a probability (2e-6 in the sums) apart."""
+    rng = np.random.default_rng(max_pos + base)
+    M = 9
+    kvk, kvv = (torch.from_numpy(_cache(rng, max_pos, Hkv, 128)).to(DEV) for _ in range(2))
+    q = _bf16(rng.standard_normal((M, Hq, 128))).to(DEV)
+
+    def attend(first, n):
+        sc = torch.empty((n, Hq, max_pos), dtype=torch.float32, device=DEV)
+        return dext.attn_decode(q[first:first + n].contiguous(), kvk, kvv,
+                                torch.tensor([base + first], dtype=torch.int32, device=DEV), sc, n)
+
+    whole = attend(0, M)
+    for first, n in ((0, 1), (4, 1), (8, 1), (0, 4), (3, 5)):
+        part = attend(first, n)
+        torch.cuda.synchronize()
+        if max_pos <= 4096:
+            assert torch.equal(part, whole[first:first + n]), (first, n)
+        else:
+            assert_close(np_(part), np_(whole[first:first + n]), what=f"tokens {first}..{first + n - 1}", rel_max=1e-5)
+
+
 @pytest.mark.parametrize("codec", [0, 1])
 def test_attn_decode_fused_split_matches_two_ops(codec):
     """Past 4096 positions mxfp4_attn_decode_fused with several tokens still
