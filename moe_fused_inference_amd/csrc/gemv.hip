@@ -453,6 +453,10 @@ __global__ __launch_bounds__(64 * R * S) void lin_small_kernel(const uint8_t* __
 //    for its own copies only.  The output's stores count in the same counter,
 //    so the wait behind them asks for a little more than the stage.
 //  * The MFMA chain of an output is lin_small_kernel<4, 1>'s: the same bits.
+//  * K is a multiple of 1024, so that a stage lies in one row tile and the bits
+//    hold, and at most 4096, so that the activation rows (16 x K / 2 bytes) leave
+//    three stages a wave of the LDS; other K have the tile per wave (stages of K
+//    512 would take 2560 and 3584 and are not tried).
 // Measured on MI355X, 151936 x 2048 from HBM, M = 8: 42.5 us for the tile per
 // wave, 34.5 us (4.8 TB/s) here.
 constexpr int kStRows = 16, kStK = 1024;                    // a stage: weight rows, K

@@ -359,8 +359,9 @@ __global__ __launch_bounds__(64 * kRtWaves) void route_scatter_kernel(const int6
 // it quantize x (four of the quantizer's blocks each).  What bounds it at these
 // sizes is latency, so a launch and the histograms' trip through memory saved
 // are worth a single workgroup's ballots (measured on MI355X, 100 tokens x 8:
-// count + scatter 4.3 + 5.4 us, 4.5 us here), which from kR1Max on are not (500
-// tokens: the call 92.0 and 90.1 us, the gain already down to 2 us).
+// count + scatter 4.3 + 5.4 us, 4.3 us here).  kR1Max is what the kR1Groups ids
+// that a lane holds come to; the gain goes down to 2 us there (500 tokens: the
+// call 92.0 and 90.1 us), so there is no longer version.
 constexpr int kR1Waves = 16, kR1Groups = 4;
 constexpr int kR1Max = 64 * kR1Waves * kR1Groups;
 
