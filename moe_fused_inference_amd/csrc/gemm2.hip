@@ -485,7 +485,9 @@ int pick_gemm2(const uint8_t* xq, const uint8_t* xsc, const uint8_t* wp, const u
     //  * else 64 x 128, three stages (two with ragged scales, to stay at two
     //    workgroups per CU): 1000 x 2000 x 2048 7.8 against 8.6 with 64 x 64, 32 x
     //    151936 x 2048 40.2 against 45.2 and 62 with 256 x 256.
-    // All tiles give the same bits (the same MFMA chain per output).
+    // (The lines for a long K and for uneven XCDs were measured on whole K steps only,
+    // and ragged ones do without them.)  All tiles give the same bits (the same MFMA
+    // chain per output).
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const int64_t t64x128 = (int64_t)((M + 63) / 64) * ((N + 127) / 128);

@@ -295,6 +295,31 @@ def test_attn_decode_split_scores_past_fp32_resolution(dext, M, Hq, Hkv, scale):
     assert_close(np_(o), ref, what=f"attn split, scores of 2^{scale}, M={M}", rel_max=1e-5)
 
 
+def test_attn_decode_split_rows_without_numbers(dext):
+    """Query rows with infinities and NaN have NaN where a token alone has it,
+    and the rows that share their tiles keep their results."""
+    rng = np.random.default_rng(3)
+    M, Hq, Hkv, max_pos, base = 3, 32, 4, 4352, 4300
+    kvk, kvv = (torch.from_numpy(_cache(rng, max_pos, Hkv, 128)).to(DEV) for _ in range(2))
+    good = _bf16(rng.standard_normal((M, Hq, 128))).to(DEV)
+    bad = good.clone()
+    bad[0, 0], bad[0, 5, 3], bad[1, 9, 7], bad[2, 31, 0] = float("nan"), float("inf"), -float("inf"), float("nan")
+    hit = torch.zeros((M, Hq), dtype=torch.bool, device=DEV)
+    hit[0, 0] = hit[0, 5] = hit[1, 9] = hit[2, 31] = True
+
+    def attend(q, first, n):
+        sc = torch.empty((n, Hq, max_pos), dtype=torch.float32, device=DEV)
+        return dext.attn_decode(q[first:first + n].contiguous(), kvk, kvv,
+                                torch.tensor([base + first], dtype=torch.int32, device=DEV), sc, n)
+
+    clean, o = attend(good, 0, M), attend(bad, 0, M)
+    alone = torch.cat([attend(bad, m, 1) for m in range(M)])
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isnan(o), torch.isnan(alone)) and torch.isnan(o[hit]).all()
+    # (a tile with an infinite reference rounds the products in the exponents of its other rows too: below 2^5 here, 2^-20)
+    assert_close(np_(o[~hit]), np_(clean[~hit]), what="rows beside", rel_max=1e-5)
+
+
 @pytest.mark.parametrize("Hq,Hkv,max_pos,base", [(32, 4, 4096, 4000), (8, 8, 4096, 63), (32, 4, 4352, 4200)])
 def test_attn_decode_token_alone_and_in_company(dext, Hq, Hkv, max_pos, base):
     """A token's result up to max_pos 4096 has the same bits in any company;
